@@ -9,6 +9,7 @@ hipcc cross-compiles for gfx950 without a GPU.  Every HIP compile line carries
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
@@ -22,7 +23,11 @@ ARCH = os.environ.get("PFDD_OFFLOAD_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = ["-O3", "-std=c++17", f"--offload-arch={ARCH}", "-fPIC", "-Wall", "-Wno-unused-function",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", f"-I{INC}", f"-I{CSRC}"]
-HIP_SOURCES = ["pfdd_api.hip"]
+# (source, object, extra flags): the reduced-basis kernels build as one unit per
+# component count and kind, in parallel with the rest
+HIP_UNITS = [("pfdd_api.hip", "pfdd_api.hip.o", [])] + [
+    ("pfdd_reduced.hip", f"pfdd_reduced_{k}{r}.o", [f"-DPFDD_RED_R={r}", f"-DPFDD_RED_KIND={k}"])
+    for k in range(4) for r in range(1, 7)] + [("pfdd_reduced.hip", "pfdd_reduced_4.o", ["-DPFDD_RED_KIND=4"])]
 C_SOURCES = ["pfdd_setup.c"]
 
 
@@ -53,15 +58,18 @@ def build(verbose=False, incremental=False):
         if incremental and _fresh(o, os.path.join(CSRC, s)):
             continue
         _run(["gcc", "-O2", "-fPIC", "-std=c99", "-Wall", f"-I{INC}", "-c", os.path.join(CSRC, s), "-o", o])
-    for s in HIP_SOURCES:
-        o = os.path.join(BUILD, s + ".o")
-        if incremental and _fresh(o, os.path.join(CSRC, s)):
-            objs.append(o)
-            continue
-        out = _run([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, s), "-o", o])
-        if verbose and out.strip():
-            print(out)
-        objs.append(o)
+
+    def compile_unit(unit):
+        src, obj, flags = unit
+        o = os.path.join(BUILD, obj)
+        if not (incremental and _fresh(o, os.path.join(CSRC, src))):
+            out = _run([HIPCC] + HIP_FLAGS + flags + ["-c", os.path.join(CSRC, src), "-o", o])
+            if verbose and out.strip():
+                print(out)
+        return o
+
+    with ThreadPoolExecutor(min(len(HIP_UNITS), os.cpu_count() or 1, 8)) as ex:
+        objs += list(ex.map(compile_unit, HIP_UNITS))
     tmp = LIB + ".tmp"
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC"] + objs + ["-o", tmp])
     os.replace(tmp, LIB)

@@ -21,6 +21,7 @@
 
 #include "pfdd_gpu.h"
 #include "pfdd_kernels.hpp"
+#include "pfdd_reduced.h"
 
 using namespace pfdd;
 
@@ -70,7 +71,7 @@ struct pfdd_ctx {
   int* step_ctr = nullptr;
   double* small = nullptr;   // reduction outputs (<= 32 doubles)
   double* avepst_d = nullptr;
-  ElasticConsts* ec = nullptr;
+  ElasticConsts* ec = nullptr;   // [0] of the eigenstrains, [1] of the reduced basis
   double* freq = nullptr;    // frec tables of the three axes, n1 + n2 + n3 doubles
   void* E6 = nullptr;        // strain spectrum [6][P], allocated on first use
   double* efield = nullptr;  // [9][P] strain/stress fields, on demand
@@ -90,6 +91,13 @@ struct pfdd_ctx {
   int il_fixed = 0;          // 1: the interleaved column kernel with compile-time S and tile (k_col_il_fixed)
   int il_fixed_row = 0;      // 1: the interleaved row kernel with compile-time S and rows (k_row_il_fixed)
   size_t c3_lds = 0;         // its dynamic LDS bytes
+  // the reduced basis (pfdd_reduced.hpp)
+  int red = 0;               // 1: the GL steps run in the reduced basis
+  int red_R = 0;             // its components
+  int red_extra = 0;         // 1: W holds the prologue's extra force, for the next step's update
+  RedArgs ra{};
+  void* Wr = nullptr;        // cx<T> [B][P][R], allocated with the first plan that uses it
+  void* Kst = nullptr;       // T [P][R(R+1)/2], K(k) in stored mode
   int plan = 0;              // the applied PFDD_PLAN_* word
   int r4 = 0;                // bit ax: radix-4 sequence for the standalone passes along axis ax
   int has_xi = 0;
@@ -423,10 +431,9 @@ int k1il_attr(pfdd_ctx* c) {
   }
 }
 
-// The row kernels write one block sum per field and row block; above this
-// many per field they are folded to FOLD in parallel before the one-block
+// The row kernels write one block sum per field and row block; above
+// FOLD_ABOVE per field they are folded to FOLD in parallel before the one-block
 // finish (128^3 x 12 FP64, 2048 per field: 0.926 -> 0.922 ms per step).
-constexpr int FOLD_ABOVE = 512;
 bool folds(const pfdd_ctx* c) { return c->row_nblk > FOLD_ABOVE; }
 
 // The gamma sums of the fused row kernel's block sums (k_finish_sums, with
@@ -619,6 +626,118 @@ int plane_launch(pfdd_ctx* c, bool finish = true, bool attr_only = false) {
   return hipPeekAtLastError() == hipSuccess ? PFDD_OK : PFDD_E_HIP;
 }
 
+// ---------------------------------------------------------------- reduced basis
+// Launches the row kernel (project: the prologue's projection of xi, without
+// an inverse transform or an update).
+template <typename T>
+int red_row(pfdd_ctx* c, bool project) {
+  RedRowLaunch<T> q{};
+  q.a = c->ra;
+  q.a.nblk = c->row_nblk;
+  q.o.mask = c->mask;
+  q.o.taupp = c->taupp;
+  q.o.extra = c->red_extra ? (const cx<T>*)c->W : nullptr;
+  q.o.project = project;
+  q.W = (cx<T>*)c->Wr;
+  q.tw = tw_of<T>(c->tw[2]);
+  q.partials = c->partials;
+  q.step_ctr = c->step_ctr;
+  q.nblk = (unsigned)c->row_nblk;
+  q.batch = (unsigned)c->B;
+  q.stream = c->stream;
+  bool ok = false;
+  with_master<T>(c, [&](auto xi) {
+    using M = decltype(xi);
+    const int n3 = c->p.n3;
+    switch (c->red_R) {
+#define PFDD_R(RR)                                                              \
+  case RR:                                                                      \
+    if constexpr (sizeof(T) == 8) ok = red_row_d##RR(q, xi, n3);                \
+    else if constexpr (lean_master<M>()) ok = red_row_l##RR(q, xi, n3);         \
+    else ok = red_row_c##RR(q, xi, n3);                                         \
+    break;
+      PFDD_R(1) PFDD_R(2) PFDD_R(3) PFDD_R(4) PFDD_R(5) PFDD_R(6)
+#undef PFDD_R
+      default: break;
+    }
+  });
+  if (!ok) return PFDD_E_RADIX;
+  return hipPeekAtLastError() == hipSuccess ? PFDD_OK : PFDD_E_HIP;
+}
+
+template <typename T>
+int red_col(pfdd_ctx* c, const FinishJob& fin = FinishJob{}) {
+  RedColLaunch<T> q{};
+  q.W = (cx<T>*)c->Wr;
+  q.ec = c->ec + 1;
+  q.Kst = (const T*)c->Kst;
+  q.P = c->P;
+  q.tw = tw_of<T>(c->tw[0]);
+  q.batch = (unsigned)c->B;
+  q.fin = fin;
+  q.stream = c->stream;
+  bool ok = false;
+  switch (c->red_R) {
+#define PFDD_R(RR)                                                \
+  case RR:                                                        \
+    if constexpr (sizeof(T) == 8) ok = red_col_d##RR(q, c->p.n1); \
+    else ok = red_col_f##RR(q, c->p.n1);                          \
+    break;
+    PFDD_R(1) PFDD_R(2) PFDD_R(3) PFDD_R(4) PFDD_R(5) PFDD_R(6)
+#undef PFDD_R
+    default: break;
+  }
+  tap(c, PFDD_STAGE_CONTRACT);
+  if (!ok) return PFDD_E_RADIX;
+  return hipPeekAtLastError() == hipSuccess ? PFDD_OK : PFDD_E_HIP;
+}
+
+template <typename T>
+int red_pass2(pfdd_ctx* c, int sign, const FoldJob& fold = FoldJob{}) {
+  RedPass2Launch<T> q{};
+  q.W = (cx<T>*)c->Wr;
+  q.outer = (long)c->B * c->p.n1;
+  q.inner = (long)c->p.n3 * c->red_R;
+  q.sign = sign;
+  q.tw = tw_of<T>(c->tw[1]);
+  q.fold = fold;
+  q.stream = c->stream;
+  bool ok;
+  if constexpr (sizeof(T) == 8) ok = red_pass2_d(q, c->p.n2);
+  else ok = red_pass2_f(q, c->p.n2);
+  tap(c, PFDD_STAGE_FFT_AXIS2);
+  if (!ok) return PFDD_E_RADIX;
+  return hipPeekAtLastError() == hipSuccess ? PFDD_OK : PFDD_E_HIP;
+}
+
+// The step: the sums of the row kernel's block sums ride along with the N2
+// pass and the column kernel, except that k_finish_sums runs by itself while
+// a point list is set (the step then reports a reduction launch, as with the
+// other plans); both add in the same order.
+template <typename T>
+int red_step(pfdd_ctx* c) {
+  int rc;
+  if ((rc = red_row<T>(c, false))) return rc;
+  tap(c, PFDD_STAGE_UPDATE);
+  c->red_extra = 0;
+  FoldJob fold{};
+  FinishJob fin{c->partials, c->hist, c->step_ctr, c->row_nblk, c->F, c->S};
+  if (folds(c)) {
+    fold = {c->partials, c->partials + c->partials_len - (size_t)c->F * FOLD, c->row_nblk, c->F};
+    fin.in = fold.out;
+    fin.nblk = FOLD;
+  }
+  if ((rc = red_pass2<T>(c, PFDD_FORWARD, fold))) return rc;
+  if (c->nline > 0) {
+    hipLaunchKernelGGL(k_finish_sums, dim3(1), dim3(FIN_THREADS), 0, c->stream, fin.in, c->F, fin.nblk, c->S, c->hist,
+                       c->step_ctr);
+    tap(c, PFDD_STAGE_FINISH);
+    fin.in = nullptr;
+  }
+  if ((rc = red_col<T>(c, fin))) return rc;
+  return red_pass2<T>(c, PFDD_BACKWARD);
+}
+
 // The N1 part of the elastic solve: forward N1, contraction, inverse N1
 // (fused into one kernel when it fits).
 // One FFT pass of W along axis ax (0: N1, 1: N2, 2: N3) for the context's
@@ -697,6 +816,7 @@ int axis3(pfdd_ctx* c, int sign) {
 template <typename T>
 int one_step(pfdd_ctx* c) {
   int rc;
+  if (c->red) return red_step<T>(c);
   if (c->plane) {
     if ((rc = plane_launch<T>(c))) return rc;
     return n1_part<T>(c, 0);
@@ -713,8 +833,34 @@ int one_step(pfdd_ctx* c) {
 }
 
 template <typename T>
+int red_prologue(pfdd_ctx* c, int quirk) {
+  int rc;
+  c->red_extra = 0;
+  if ((rc = red_row<T>(c, true))) return rc;
+  if ((rc = red_pass2<T>(c, PFDD_FORWARD))) return rc;
+  if ((rc = red_col<T>(c))) return rc;
+  if ((rc = red_pass2<T>(c, PFDD_BACKWARD))) return rc;
+  if (!quirk) return PFDD_OK;
+  // virtualevolv's term couples each field with itself only, so it has no
+  // form in the components: its force goes to W, per field in real space,
+  // and the first update adds it
+  const long n = (long)c->F * c->P;
+  hipLaunchKernelGGL((k_xi_to_w<T>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, xm<T>(c),
+                     (cx<T>*)c->W, n);
+  for (int ax = 2; ax >= 0; ax--)
+    if ((rc = pass<T>(c, ax, PFDD_FORWARD))) return rc;
+  hipLaunchKernelGGL((k_diag_dd<T>), dim3((unsigned)((c->P + 255) / 256), (unsigned)c->B), dim3(256), 0, c->stream,
+                     (cx<T>*)c->W, c->ec, c->P);
+  for (int ax = 0; ax <= 2; ax++)
+    if ((rc = pass<T>(c, ax, PFDD_BACKWARD))) return rc;
+  c->red_extra = 1;
+  return PFDD_OK;
+}
+
+template <typename T>
 int prologue(pfdd_ctx* c, int quirk) {
   int rc;
+  if (c->red) return red_prologue<T>(c, quirk);
   const long n = (long)c->F * c->P;
   if (c->il)
     hipLaunchKernelGGL((k_xi_to_w_il<T>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, xm<T>(c),
@@ -828,6 +974,104 @@ void cijkl(double C[81], double C11, double C12, double C44) {
         }
 }
 
+// Row a of the strain constants: s_a = C:e_a, its trace sum, and the six
+// symmetric components (00, 01, 02, 11, 12, 22) of s_a and of w_t sym(e_a)_t / mu.
+void set_strain_consts(ElasticConsts& h, int a, const double e9[9]) {
+  const int ti[6] = {0, 0, 0, 1, 1, 2}, tj[6] = {0, 1, 2, 1, 2, 2};
+  for (int ij = 0; ij < 9; ij++) h.eps[a][ij] = e9[ij];
+  double ts = 0.0;
+  for (int ij = 0; ij < 9; ij++) {
+    double s = 0.0;
+    for (int mn = 0; mn < 9; mn++) s += h.C[ij * 9 + mn] * h.eps[a][mn];
+    h.sig[a][ij] = s;
+    ts += s;
+  }
+  h.Tsum[a] = ts;
+  for (int t = 0; t < 6; t++) {
+    const int i = ti[t], j = tj[t];
+    h.sig6[a][t] = 0.5 * (h.sig[a][3 * i + j] + h.sig[a][3 * j + i]);
+    h.e6m[a][t] = (i == j ? 1.0 : 2.0) * 0.5 * (h.eps[a][3 * i + j] + h.eps[a][3 * j + i]) * h.inv_mu;
+    h.sig6f[a][t] = (float)h.sig6[a][t];
+    h.e6mf[a][t] = (float)h.e6m[a][t];
+  }
+}
+
+// s_a:e_b for the first S rows.
+void set_pair_consts(ElasticConsts& h, int S) {
+  for (int a = 0; a < S; a++)
+    for (int b = 0; b < S; b++) {
+      double se = 0.0;
+      for (int mn = 0; mn < 9; mn++) se += h.sig[a][mn] * h.eps[b][mn];
+      h.SE[a][b] = se;
+    }
+}
+
+// The reduced basis of the context's eigenstrains: an orthonormal basis of
+// the span of their symmetric parts (inner product x:y over all nine
+// components) by Gram-Schmidt with the largest remainder first, each vector
+// orthogonalised twice, in long double.  A remainder below 8 ulp of the
+// largest strain is rounding of the strains themselves.  With R = S the
+// strains are the basis.  `k` starts as the context's constants and gets the
+// basis strains in the place of the eigenstrains.
+void make_basis(pfdd_ctx* c, ElasticConsts& k) {
+  const int S = c->S;
+  const int ti[6] = {0, 0, 0, 1, 1, 2}, tj[6] = {0, 1, 2, 1, 2, 2};
+  const long double w6[6] = {1, 2, 2, 1, 2, 1};
+  long double e6[MAXS][6], rem[MAXS][6], h[RED_MAXR][6];
+  auto dot = [&](const long double* x, const long double* y) {
+    long double v = 0;
+    for (int t = 0; t < 6; t++) v += w6[t] * x[t] * y[t];
+    return v;
+  };
+  long double top = 0;
+  for (int a = 0; a < S; a++) {
+    for (int t = 0; t < 6; t++)
+      rem[a][t] = e6[a][t] = 0.5L * ((long double)c->p.eps[a][ti[t]][tj[t]] + (long double)c->p.eps[a][tj[t]][ti[t]]);
+    top = std::max(top, dot(e6[a], e6[a]));
+  }
+  const long double floor2 = top * 8 * 8 * 0x1p-104L;
+  int R = 0;
+  while (R < RED_MAXR && R < S) {
+    int best = 0;
+    for (int a = 1; a < S; a++)
+      if (dot(rem[a], rem[a]) > dot(rem[best], rem[best])) best = a;
+    const long double d2 = dot(rem[best], rem[best]);
+    if (!(d2 > floor2) && R > 0) break;
+    const long double inv = d2 > 0 ? 1 / sqrtl(d2) : 0;
+    for (int t = 0; t < 6; t++) h[R][t] = rem[best][t] * inv;
+    R++;
+    for (int a = 0; a < S; a++)
+      for (int pass = 0; pass < 2; pass++)
+        for (int q = 0; q < R; q++) {
+          const long double v = dot(h[q], rem[a]);
+          for (int t = 0; t < 6; t++) rem[a][t] -= v * h[q][t];
+        }
+  }
+  RedArgs& ra = c->ra;
+  for (int a = 0; a < S; a++)
+    for (int q = 0; q < R; q++) ra.al[a][q] = R == S ? (a == q ? 1.0 : 0.0) : (double)dot(h[q], e6[a]);
+  ra.P = c->P;
+  ra.S = S;
+  ra.uq2 = c->p.uq2;
+  ra.two_pi = 2.0 * c->p.pi_const;
+  ra.inv_n = 1.0 / (double)c->P;
+  for (int a = 0; a < S; a++) {
+    ra.cd2[a] = c->p.cd2[a];
+    ra.asf_pi[a] = c->p.asf2[a] * c->p.pi_const;
+    ra.dslip[a] = c->p.dslip[a];
+  }
+  ra.tau = c->taud;
+  for (int q = 0; q < R; q++) {
+    double e9[9];
+    for (int t = 0; t < 6; t++)
+      e9[3 * ti[t] + tj[t]] = e9[3 * tj[t] + ti[t]] = (double)(R == S ? e6[q][t] : h[q][t]);
+    set_strain_consts(k, q, e9);
+  }
+  set_pair_consts(k, R);
+  k.ns = R;
+  c->red_R = R;
+}
+
 template <typename T>
 void* dev_alloc(size_t bytes, long long& total) {
   void* p = nullptr;
@@ -938,7 +1182,7 @@ void pfdd_destroy(pfdd_ctx* c) {
   if (c->graph) (void)hipGraphExecDestroy(c->graph);
   void* bufs[] = {c->xi,   c->W,        c->Bsym, c->mask, c->taupp, c->taud,   c->partials, c->hist,
                   c->step_ctr, c->small, c->avepst_d, c->ec, c->E6,  c->efield, c->sfield,   c->freq,
-                  c->line_pts, c->line_out};
+                  c->line_pts, c->line_out, c->Wr, c->Kst};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   for (auto& t : c->tw) {
@@ -1019,6 +1263,68 @@ void drop_graph(pfdd_ctx* c) {
   }
 }
 
+// B(k) in stored mode, on the first plan that reads it.
+int build_stored(pfdd_ctx* c) {
+  const size_t rsz = c->fp64 ? sizeof(double) : sizeof(float);
+  const long P = c->P;
+  const int S = c->S;
+  if (!(c->Bsym = dev_alloc<char>(rsz * c->ntri * P, c->bytes))) return PFDD_E_ALLOC;
+  const unsigned nb = (unsigned)((P + 255) / 256);
+#define PFDD_BB(T, SM) hipLaunchKernelGGL((k_build_B<T, SM>), dim3(nb), dim3(256), 0, c->stream, (T*)c->Bsym, c->ec, P)
+  if (c->fp64) {
+    if (S <= 4) PFDD_BB(double, 4); else if (S <= 8) PFDD_BB(double, 8); else PFDD_BB(double, 16);
+  } else {
+    if (S <= 4) PFDD_BB(float, 4); else if (S <= 8) PFDD_BB(float, 8); else PFDD_BB(float, 16);
+  }
+#undef PFDD_BB
+  return hipPeekAtLastError() == hipSuccess ? PFDD_OK : PFDD_E_HIP;
+}
+
+// Whether AUTO runs the steps in the reduced basis: wherever the fused row
+// and column lengths exist.
+bool auto_reduced(const pfdd_ctx* c, int plan) {
+  const pfdd_params& p = c->p;
+  if (plan != PFDD_PLAN_AUTO || !fused_len(p.n1) || !fused_len(p.n3)) return false;
+  const size_t csz = c->fp64 ? sizeof(double2) : sizeof(float2);
+  if (!c->stored && p.n1 == p.n3 && il_fixed_S(p.n1) == c->S && csz * c->S * c->P <= (128u << 20)) return false;
+  return true;
+}
+
+// The work array of the reduced basis (and K(k) in stored mode), on first
+// use; false when the memory for it is not there (the caller then takes a
+// plan without it).
+bool ensure_reduced(pfdd_ctx* c) {
+  if (c->Wr) return true;
+  const size_t csz = c->fp64 ? sizeof(double2) : sizeof(float2);
+  const int R = c->red_R;
+  long long bytes = 0;
+  void* wr = dev_alloc<char>(csz * c->B * c->P * R, bytes);
+  void* ks = c->stored && wr ? dev_alloc<char>(csz / 2 * (R * (R + 1) / 2) * c->P, bytes) : nullptr;
+  bool ok = wr && (ks || !c->stored) && red_pass2_attr(c->p.n2);
+  if (ok && ks) {
+    switch (R) {
+#define PFDD_R(RR)                                                             \
+  case RR:                                                                     \
+    if (c->fp64) red_build_d##RR((double*)ks, c->ec + 1, c->P, c->stream);     \
+    else red_build_f##RR((float*)ks, c->ec + 1, c->P, c->stream);              \
+    break;
+      PFDD_R(1) PFDD_R(2) PFDD_R(3) PFDD_R(4) PFDD_R(5) PFDD_R(6)
+#undef PFDD_R
+    }
+    ok = hipPeekAtLastError() == hipSuccess;
+  }
+  if (!ok) {
+    if (wr) (void)hipFree(wr);
+    if (ks) (void)hipFree(ks);
+    (void)hipGetLastError();
+    return false;
+  }
+  c->Wr = wr;
+  c->Kst = ks;
+  c->bytes += bytes;
+  return true;
+}
+
 // Kernel choice for a plan word (PFDD_E_SHAPE when a requested tile does not
 // fit).  The state of W between steps depends on the kernels, so a new
 // prologue is needed afterwards.
@@ -1042,6 +1348,23 @@ int apply_plan(pfdd_ctx* c, int plan) {
     c->plan = plan;
     c->prologue_done = 0;
     return PFDD_OK;
+  }
+  c->red = 0;
+  if (auto_reduced(c, plan) && ensure_reduced(c)) {
+    c->r4 = 0;
+    c->row_tile = c->c3_tile = 0;
+    c->c3_lds = 0;
+    c->plane = c->il = c->il_fixed = c->il_fixed_row = 0;
+    c->row_nblk = p.n1 * p.n2 / red_rows(p.n3);
+    c->red = 1;
+    drop_graph(c);
+    c->plan = plan;
+    c->prologue_done = 0;
+    return PFDD_OK;
+  }
+  if (c->stored && !c->Bsym) {
+    const int rc = build_stored(c);
+    if (rc) return rc;
   }
   // AUTO takes the interleaved layout where its compile-time row and column
   // kernels exist (S = 12 at N1 = N3 = 128 or 256, S = 3 at 512; recomputed
@@ -1196,7 +1519,6 @@ int ctx_create(const pfdd_params* p, int batch, hipStream_t shared, pfdd_ctx** o
       FAIL(PFDD_E_HIP);
     }
     const size_t csz = c->fp64 ? sizeof(double2) : sizeof(float2);
-    const size_t rsz = c->fp64 ? sizeof(double) : sizeof(float);
     const long P = c->P;
     const int S = c->S, F = c->F;
     const int ns3[3] = {p->n1, p->n2, p->n3};
@@ -1215,7 +1537,7 @@ int ctx_create(const pfdd_params* p, int batch, hipStream_t shared, pfdd_ctx** o
     if (!(c->step_ctr = (int*)dev_alloc<char>(sizeof(int) * 4, c->bytes))) FAIL(PFDD_E_ALLOC);
     if (!(c->small = (double*)dev_alloc<char>(sizeof(double) * 32, c->bytes))) FAIL(PFDD_E_ALLOC);
     if (!(c->avepst_d = (double*)dev_alloc<char>(sizeof(double) * 9, c->bytes))) FAIL(PFDD_E_ALLOC);
-    if (!(c->ec = (ElasticConsts*)dev_alloc<char>(sizeof(ElasticConsts), c->bytes))) FAIL(PFDD_E_ALLOC);
+    if (!(c->ec = (ElasticConsts*)dev_alloc<char>(2 * sizeof(ElasticConsts), c->bytes))) FAIL(PFDD_E_ALLOC);
     if (!(c->taud = (double2*)dev_alloc<char>(sizeof(double2) * F, c->bytes))) FAIL(PFDD_E_ALLOC);
     if (hipMemsetAsync(c->step_ctr, 0, sizeof(int) * 4, c->stream) != hipSuccess) FAIL(PFDD_E_HIP);
     if (hipMemsetAsync(c->xi, 0, c->xi_bytes, c->stream) != hipSuccess) FAIL(PFDD_E_HIP);
@@ -1232,7 +1554,9 @@ int ctx_create(const pfdd_params* p, int batch, hipStream_t shared, pfdd_ctx** o
             goto fail;
     }
     // elastic constants (Bmatrix G.c:340-358; s_a = C:e_a etc.)
-    ElasticConsts h{};
+    // two sets: of the eigenstrains, and of the reduced basis
+    std::vector<ElasticConsts> both(2);
+    ElasticConsts& h = both[0];
     h.mu = p->C44;
     h.ll = p->C12;
     h.mup = p->C11 - p->C12 - 2 * p->C44;
@@ -1244,33 +1568,11 @@ int ctx_create(const pfdd_params* p, int batch, hipStream_t shared, pfdd_ctx** o
       h.T[pq] = t;
     }
     for (int a = 0; a < S; a++) {
-      for (int ij = 0; ij < 9; ij++) h.eps[a][ij] = p->eps[a][ij / 3][ij % 3];
-      double ts = 0.0;
-      for (int ij = 0; ij < 9; ij++) {
-        double s = 0.0;
-        for (int mn = 0; mn < 9; mn++) s += h.C[ij * 9 + mn] * h.eps[a][mn];
-        h.sig[a][ij] = s;
-        ts += s;
-      }
-      h.Tsum[a] = ts;
+      double e9[9];
+      for (int ij = 0; ij < 9; ij++) e9[ij] = p->eps[a][ij / 3][ij % 3];
+      set_strain_consts(h, a, e9);
     }
-    {  // six symmetric components (00, 01, 02, 11, 12, 22) of s_b and of w_t sym(e_a)_t / mu
-      const int ti[6] = {0, 0, 0, 1, 1, 2}, tj[6] = {0, 1, 2, 1, 2, 2};
-      for (int a = 0; a < S; a++)
-        for (int t = 0; t < 6; t++) {
-          const int i = ti[t], j = tj[t];
-          h.sig6[a][t] = 0.5 * (h.sig[a][3 * i + j] + h.sig[a][3 * j + i]);
-          h.e6m[a][t] = (i == j ? 1.0 : 2.0) * 0.5 * (h.eps[a][3 * i + j] + h.eps[a][3 * j + i]) * h.inv_mu;
-          h.sig6f[a][t] = (float)h.sig6[a][t];
-          h.e6mf[a][t] = (float)h.e6m[a][t];
-        }
-    }
-    for (int a = 0; a < S; a++)
-      for (int b = 0; b < S; b++) {
-        double se = 0.0;
-        for (int mn = 0; mn < 9; mn++) se += h.sig[a][mn] * h.eps[b][mn];
-        h.SE[a][b] = se;
-      }
+    set_pair_consts(h, S);
     h.d[0] = p->d1; h.d[1] = p->d2; h.d[2] = p->d3;
     // frec (G.c:2698-2741) per axis, evaluated with the same arithmetic as the reference
     std::vector<double> fr((size_t)p->n1 + p->n2 + p->n3);
@@ -1293,7 +1595,10 @@ int ctx_create(const pfdd_params* p, int batch, hipStream_t shared, pfdd_ctx** o
     h.g_iso = (h.mu + h.ll) / (h.mu * h.mu * (1.0 + (h.mu + h.ll) / h.mu));
     h.n[0] = p->n1; h.n[1] = p->n2; h.n[2] = p->n3;
     h.ns = S;
-    if (hipMemcpyAsync(c->ec, &h, sizeof(h), hipMemcpyHostToDevice, c->stream) != hipSuccess) FAIL(PFDD_E_HIP);
+    both[1] = h;
+    make_basis(c, both[1]);
+    if (hipMemcpyAsync(c->ec, both.data(), 2 * sizeof(h), hipMemcpyHostToDevice, c->stream) != hipSuccess)
+      FAIL(PFDD_E_HIP);
     if (hipStreamSynchronize(c->stream) != hipSuccess) FAIL(PFDD_E_HIP);
     // step arguments
     c->sa.P = P;
@@ -1309,18 +1614,6 @@ int ctx_create(const pfdd_params* p, int batch, hipStream_t shared, pfdd_ctx** o
       c->sa.dslip[a] = p->dslip[a];
     }
     c->sa.tau = c->taud;
-    if (c->stored) {
-      if (!(c->Bsym = dev_alloc<char>(rsz * c->ntri * P, c->bytes))) FAIL(PFDD_E_ALLOC);
-      const unsigned nb = (unsigned)((P + 255) / 256);
-#define PFDD_BB(T, SM) hipLaunchKernelGGL((k_build_B<T, SM>), dim3(nb), dim3(256), 0, c->stream, (T*)c->Bsym, c->ec, P)
-      if (c->fp64) {
-        if (S <= 4) PFDD_BB(double, 4); else if (S <= 8) PFDD_BB(double, 8); else PFDD_BB(double, 16);
-      } else {
-        if (S <= 4) PFDD_BB(float, 4); else if (S <= 8) PFDD_BB(float, 8); else PFDD_BB(float, 16);
-      }
-#undef PFDD_BB
-      if (hipPeekAtLastError() != hipSuccess) FAIL(PFDD_E_HIP);
-    }
     if ((rc = apply_plan(c, p->plan))) goto fail;
     if (hipStreamSynchronize(c->stream) != hipSuccess) FAIL(PFDD_E_HIP);
   }
@@ -1515,6 +1808,13 @@ int run_steps(pfdd_ctx* const* cs, int nc, hipStream_t st, hipGraphExec_t* graph
       hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, st, cs[i]->step_ctr, 0);
     HIPCK(hipPeekAtLastError());
     int left = chunk;
+    bool first = false;  // the first step after a prologue may take an argument that the others do not
+    for (int i = 0; i < nc; i++) first = first || cs[i]->red_extra;
+    if (first) {
+      const int rc = one();
+      if (rc) return rc;
+      left--;
+    }
     if (left >= GRAPH_STEPS && !*graph) {
       hipGraph_t g;
       HIPCK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
@@ -1581,7 +1881,7 @@ std::vector<int> plan_candidates(pfdd_ctx* c) {
   const int saved = c->plan;
   auto add = [&](int plan) {
     if (apply_plan(c, plan) != PFDD_OK) return;
-    const long sig = ((long)c->row_tile << 32) | ((long)c->c3_tile << 8) | (c->il << 1) | c->plane;
+    const long sig = ((long)c->red << 60) | ((long)c->row_tile << 32) | ((long)c->c3_tile << 8) | (c->il << 1) | c->plane;
     for (long v : seen)
       if (v == sig) return;
     seen.push_back(sig);
@@ -1688,7 +1988,7 @@ int autotune_ctx(pfdd_ctx* c, int steps, int* best_plan, float* best_ms) {
     // stage 2: radix-4 sequences for the standalone passes the best plan uses
     if ((rc = apply_plan(c, best))) break;
     const int n3[3] = {c->p.n1, c->p.n2, c->p.n3};
-    const bool standalone[3] = {c->c3_tile == 0, !c->plane, !c->plane && c->row_tile == 0};
+    const bool standalone[3] = {!c->red && c->c3_tile == 0, !c->plane, !c->red && !c->plane && c->row_tile == 0};
     const int bit[3] = {PFDD_PLAN_RADIX4_AXIS1, PFDD_PLAN_RADIX4_AXIS2, PFDD_PLAN_RADIX4_AXIS3};
     int axes = 0;
     for (int ax = 0; ax < 3; ax++)
@@ -1883,10 +2183,13 @@ int enqueue_stage(pfdd_ctx* c, int stage, int reps) {
     const int sign = (r & 1) ? PFDD_BACKWARD : PFDD_FORWARD;
     switch (stage) {
       case PFDD_STAGE_UPDATE:
-        rc = c->plane ? plane_launch<T>(c, false) : c->row_tile > 0 ? k1_launch<T>(c, false) : update<T>(c, false);
+        rc = c->red            ? red_row<T>(c, false)
+             : c->plane        ? plane_launch<T>(c, false)
+             : c->row_tile > 0 ? k1_launch<T>(c, false)
+                               : update<T>(c, false);
         break;
       case PFDD_STAGE_FINISH:
-        if (!c->plane && c->row_tile > 0)
+        if (c->red || (!c->plane && c->row_tile > 0))
           finish_rows(c, nullptr);
         else
           hipLaunchKernelGGL(k_finish_sums, dim3(1), dim3(FIN_THREADS), 0, c->stream, c->partials, c->F,
@@ -1897,13 +2200,13 @@ int enqueue_stage(pfdd_ctx* c, int stage, int reps) {
         rc = pass<T>(c, 2, sign);
         break;
       case PFDD_STAGE_FFT_AXIS2:
-        rc = pass<T>(c, 1, sign);
+        rc = c->red ? red_pass2<T>(c, sign) : pass<T>(c, 1, sign);
         break;
       case PFDD_STAGE_FFT_AXIS1:
         rc = pass<T>(c, 0, sign);
         break;
       case PFDD_STAGE_CONTRACT:
-        rc = c->c3_tile > 0 ? k3_launch<T>(c, 0) : contract<T>(c, 0);
+        rc = c->red ? red_col<T>(c) : c->c3_tile > 0 ? k3_launch<T>(c, 0) : contract<T>(c, 0);
         break;
       case PFDD_STAGE_STEP:
         hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, c->stream, c->step_ctr, 0);
@@ -1924,7 +2227,7 @@ int enqueue_stage(pfdd_ctx* c, int stage, int reps) {
 
 extern "C" int pfdd_step_plan(const pfdd_ctx* c, int* launches) {
   if (!c || !launches) return PFDD_E_SHAPE;
-  const bool r = c->row_tile > 0 || c->plane, k3 = c->c3_tile > 0;
+  const bool r = c->row_tile > 0 || c->plane || c->red, k3 = c->c3_tile > 0 || c->red;
   launches[PFDD_STAGE_UPDATE] = 1;
   launches[PFDD_STAGE_FFT_AXIS3] = r ? 0 : 2;
   launches[PFDD_STAGE_FFT_AXIS2] = c->plane ? 0 : 2;
@@ -1933,7 +2236,8 @@ extern "C" int pfdd_step_plan(const pfdd_ctx* c, int* launches) {
   launches[PFDD_STAGE_STEP] = 0;
   launches[PFDD_STAGE_COPY] = 0;
   // + the fold of the row kernel's block sums when there are many, + the line sums while a list is set
-  launches[PFDD_STAGE_FINISH] = 1 + (folds(c) ? 1 : 0) + (c->nline > 0 ? 1 : 0);
+  // (reduced basis: inside the other launches, unless a list is set)
+  launches[PFDD_STAGE_FINISH] = c->red ? (c->nline > 0 ? 2 : 0) : 1 + (folds(c) ? 1 : 0) + (c->nline > 0 ? 1 : 0);
   return PFDD_OK;
 }
 

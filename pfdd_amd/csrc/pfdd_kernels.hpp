@@ -480,7 +480,7 @@ __device__ __forceinline__ void finish_body(const double* __restrict__ partials,
 // j-th of FOLD consecutive ranges of field f's block sums in a fixed order,
 // giving FOLD sums per field for k_finish_sums.
 constexpr int FOLD = 16;
-__global__ void __launch_bounds__(256)
+static __global__ void __launch_bounds__(256)
 k_fold_partials(const double* __restrict__ in, int nblk, double* __restrict__ out) {
   __shared__ double red[256 / 64];
   const int f = blockIdx.y, j = blockIdx.x;
@@ -492,7 +492,7 @@ k_fold_partials(const double* __restrict__ in, int nblk, double* __restrict__ ou
   if (threadIdx.x == 0) out[(long)f * FOLD + j] = s;
 }
 
-__global__ void __launch_bounds__(FIN_THREADS)
+static __global__ void __launch_bounds__(FIN_THREADS)
 k_finish_sums(const double* __restrict__ partials, int nfields, int nblk, int ns, double* out, int* step_ctr) {
   __shared__ double fsum[FIN_MAX_FIELDS];
   finish_body(partials, nfields, nblk, ns, out, step_ctr, fsum);
@@ -578,7 +578,7 @@ __global__ void k_xi_to_w(Master<T> xi, cx<T>* __restrict__ W, long n) {
   }
 }
 
-__global__ void k_set_int(int* p, int v) {
+static __global__ void k_set_int(int* p, int v) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *p = v;
 }
 
@@ -799,6 +799,34 @@ __device__ __forceinline__ void contract_point(const cx<T> (&v)[SM], const Elast
   }
 }
 
+// The prologue's extra term alone (virtualevolv G.c:1426-1441): every
+// spectrum value v_a times sum_ij DD_a,ij.  Field-major W; grid = (points, instances).
+template <typename T>
+__global__ void __launch_bounds__(256)
+k_diag_dd(cx<T>* __restrict__ W, const ElasticConsts* __restrict__ ec, long P) {
+  const long pt = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (pt >= P) return;
+  const int S = ec->ns;
+  W += (long)blockIdx.y * S * P + pt;
+  double f[3], g[6];
+  kvec(pt, ec, f);
+  const bool nz = green6(f, ec, g);
+  const double* t9 = ec->T;
+  const double tf[3] = {t9[0] * f[0] + t9[1] * f[1] + t9[2] * f[2], t9[3] * f[0] + t9[4] * f[1] + t9[5] * f[2],
+                        t9[6] * f[0] + t9[7] * f[1] + t9[8] * f[2]};
+  for (int a = 0; a < S; a++) {
+    T dd = (T)0;
+    if (nz) {
+      double u[3], gu[3];
+      sig_f(ec, a, f, u);
+      gmul(g, u, gu);
+      dd = (T)((ec->Tsum[a] - (gu[0] * tf[0] + gu[1] * tf[1] + gu[2] * tf[2])) * ec->inv_mu);
+    }
+    const cx<T> v = W[(long)a * P];
+    W[(long)a * P] = {v.x * dd, v.y * dd};
+  }
+}
+
 // Pointwise contraction in place on W (used when the fused column kernel
 // does not fit).
 // IL: the interleaved layout (fields of a point together).
@@ -839,7 +867,7 @@ k_contract(cx<T>* __restrict__ W, const T* __restrict__ Bsym, const ElasticConst
 // change a bit.  fourn runs the axes N3, N2, N1 in both directions.
 // One block per line.
 constexpr int FOURN_THREADS = 256;
-__global__ void __launch_bounds__(FOURN_THREADS)
+static __global__ void __launch_bounds__(FOURN_THREADS)
 k_fourn_axis(cx<float>* __restrict__ data, long inner, int n, int logn, const float2* __restrict__ tw) {
 #pragma clang fp contract(off)
   __shared__ cx<float> sm[1024];
@@ -1127,7 +1155,7 @@ k_row_step_il(cx<T>* __restrict__ W, M xi, const uint8_t* __restrict__ mask,
   constexpr int TPP = make_plan(N).tpp, LD = pitch<N>();
   extern __shared__ unsigned char lds_raw[];
   cx<T>* sm = reinterpret_cast<cx<T>*>(lds_raw);
-  const int S = a.ns, npen = S * R, NT = blockDim.x;
+  const int S = a.ns, npen = S * R;
   double* red = reinterpret_cast<double*>(sm + (long)npen * LD);
   __shared__ cx<T> twl[N];
   stage_twiddles<T, N>(twl, tw);
@@ -1742,7 +1770,7 @@ struct EnsDev {
   EnsClassDev cls[ENS_MAX_CLASSES];
 };
 
-__global__ void k_ens_reset(int* q) {
+static __global__ void k_ens_reset(int* q) {
   if (threadIdx.x < ENS_Q_INTS && threadIdx.x != 1) q[threadIdx.x] = 0;
 }
 

@@ -1,0 +1,401 @@
+// pfdd_reduced.hpp -- the GL step in a reduced basis of the eigenstrains.
+//
+// The interaction matrix depends on the slip systems only through the
+// symmetric parts of their eigenstrains: B_ab(k) = e_a : L(k) : e_b / mu with
+// one fourth-order kernel L(k) = C - C.f G f.C for all pairs (Bmatrix,
+// G.c:386-402).  The symmetric parts of S eigenstrains span R <= min(S, 6)
+// dimensions (5 for the 12 FCC systems, whose strains are traceless; 2 for
+// the three systems of one slip plane).  With a basis h_t of that span,
+// e_a = sum_t al_at h_t,
+//   sum_b B_ab xi_b^ = sum_t al_at [ sum_u K_tu(k) c_u^ ],
+//   c_u = sum_b al_bu xi_b,   K_tu = h_t : L : h_u / mu,
+// and the sums over a and b commute with the Fourier transform.  So a step
+// transforms R component fields instead of S slip fields: the row kernel
+// forms them from xi in real space right after the update, and expands the R
+// transformed results to the S driving forces right before it.
+//
+// What bounds the step is memory traffic: per point 32 S + 32 R bytes in the
+// row kernel and 3 x 32 R in the two N2 passes and the column kernel (FP64),
+// against 160 S to 224 S with the transforms on the slip fields.  Measured per
+// GL step, slip fields -> components: 128^3 x 12 FP64 682 -> 358 us, lean 346
+// -> 218, 96^3 x 3 lean 121 -> 70, 256x256x192 x 3 FP64 1467 -> 836, 32^3 x 3
+// FP64 33 -> 18; 256x256x128 x 12 mixed with stored B 3240 -> 1103 (15 stored
+// values a k-point instead of 78).
+//
+// Layout: W[instance][N1][N2][N3][R], the components of a point together.
+#pragma once
+#include "pfdd_kernels.hpp"
+
+namespace pfdd {
+
+constexpr int RED_MAXR = 6;
+
+// What the row kernel needs of the step (by value, read through the scalar cache).
+struct RedArgs {
+  long P;
+  int S;
+  int nblk;                    // row blocks per field
+  double uq2, two_pi, inv_n;
+  double cd2[MAXS], asf_pi[MAXS], dslip[MAXS];
+  double al[MAXS][RED_MAXR];   // e_a = sum_t al[a][t] h_t
+  const double2* tau;          // per field: (tau, rate)
+};
+// Options of the general variant (OPT): frozen points, per-point shear, the
+// prologue's extra force (virtualevolv G.c:1426-1447, per field in real
+// space), and the projection alone (the prologue: no inverse transform, no
+// update).  Null pointers switch the first three off.
+template <typename T> struct RedOpt {
+  const uint8_t* mask;
+  const double* taupp;
+  const cx<T>* extra;
+  int project;
+};
+
+// ---------------------------------------------------------------- wave sums
+template <int CTRL> __device__ __forceinline__ double dpp_mov(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// Sums of four values over a wave at once: lane l with l % 4 = j returns the
+// sum of v[j].  Each of the first two exchanges halves the values a lane
+// carries, so four sums take 33 vector instructions and 4 LDS permutes
+// instead of 4 x 18 and 4 x 4.
+__device__ __forceinline__ double wave_sum4(const double (&v)[4]) {
+  const bool b0 = threadIdx.x & 1, b1 = threadIdx.x & 2;
+  double k0 = (b0 ? v[1] : v[0]) + dpp_mov<0xB1>(b0 ? v[0] : v[1]);  // quad_perm 1,0,3,2
+  double k1 = (b0 ? v[3] : v[2]) + dpp_mov<0xB1>(b0 ? v[2] : v[3]);
+  double k = (b1 ? k1 : k0) + dpp_mov<0x4E>(b1 ? k0 : k1);           // quad_perm 2,3,0,1
+  k += dpp_mov<0x124>(k);                                            // row_ror 4
+  k += dpp_mov<0x128>(k);                                            // row_ror 8
+  k += __shfl_xor(k, 16, 64);
+  k += __shfl_xor(k, 32, 64);
+  return k;
+}
+
+// ---------------------------------------------------------------- row kernel
+// Rows per block: about 256 points, one per thread.
+constexpr int red_rows(int n) { return n <= 64 ? (n <= 32 ? 4 : n == 48 ? 4 : 4) : n <= 128 ? 2 : 1; }
+template <typename T, int N, int R> struct RowRed {
+  static constexpr int ROWS = red_rows(N), NT = ROWS * N, TPP = make_plan(N).tpp;
+  static constexpr int SH = 3, LD = padded_pitch<N, SH>(), NPEN = ROWS * R;
+};
+
+// A pencil of the interleaved array as one thread sees it: element i at p[i * stride].
+template <typename T> struct StridedPencil {
+  cx<T>* p;
+  long stride;
+  static constexpr bool in_lds = false;
+  __device__ __forceinline__ cx<T> load(int, int i) const { return p[i * stride]; }
+  __device__ __forceinline__ void store(int, int i, cx<T> v) const { p[i * stride] = v; }
+};
+
+// plasticevolv (G.c:3485-3489) with the shear already divided by dslip.
+template <bool F32SIN>
+__device__ __forceinline__ void gl_point_q(double2& x, double dre, double dim, double cd2, double asf_pi, double tq,
+                                           const RedArgs& a) {
+  const double arg = a.two_pi * x.x;
+  double sn;
+  if constexpr (F32SIN) {
+    constexpr double TWO_PI_HI = 6.283185307179586, TWO_PI_LO = 2.4492935982947064e-16;
+    const double k = rint(arg * (1.0 / TWO_PI_HI));
+    sn = (double)sinf((float)fma(-k, TWO_PI_LO, fma(-k, TWO_PI_HI, arg)));
+  } else {
+    sn = sin(arg);
+  }
+  x.x -= cd2 * (a.uq2 * dre * a.inv_n + asf_pi * sn - tq);
+  x.y -= a.uq2 * cd2 * (dim * a.inv_n);
+}
+
+// One block: ROWS rows along N3 of all R components.  Inverse N3 transform
+// (G.c:4638), then one point per thread: the S driving forces from the R
+// components, plasticevolv (G.c:3470-3501) on the S fields of the point, the
+// new components from them, the fields' sums of Re xi / P; forward N3
+// transform (first pass of G.c:4599).  The first pass reads W into registers
+// and the last writes it back.  grid = (row blocks, instances).
+template <typename T, int N, int R, typename M, bool OPT>
+__global__ void __launch_bounds__((RowRed<T, N, R>::NT))
+k_row_red(cx<T>* __restrict__ W, M xi, const RedArgs a, const RedOpt<T> o, const cx<T>* __restrict__ tw,
+          double* __restrict__ partials, const int* __restrict__ step_ctr) {
+  using K = RowRed<T, N, R>;
+  constexpr int NT = K::NT, LD = K::LD, TPP = K::TPP, SH = K::SH, ROWS = K::ROWS, CH = 4;
+  static_assert(NT % 64 == 0 && R * TPP <= N, "one pencil per lane group");
+  __shared__ cx<T> sm[K::NPEN * LD];
+  __shared__ cx<T> twl[N];
+  __shared__ double tq[MAXS], wred[NT / 64][MAXS];
+  const int t = threadIdx.x, S = a.S, inst = blockIdx.y;
+  const long blk = blockIdx.x, P = a.P, pt0 = blk * NT;
+  // FFT lanes: component fastest, then the lane within the pencil, then the row
+  const int fc = t % R, fq = (t / R) % TPP, fr = t / (R * TPP);
+  const int pen = fr < ROWS ? fr * R + fc : 1 << 30;
+  const StridedPencil<T> g{W + ((long)inst * P + pt0 + (long)fr * N) * R + fc, R};
+  const LdsPencils<T, SH> l{sm, LD};
+  TwStage<T, N, NT> ts;
+  ts.load(tw);
+  const long xo = (long)inst * S * P + pt0 + t;  // this thread's point of field 0
+  typename M::Raw cur[CH], nxt[CH];
+#pragma unroll
+  for (int j = 0; j < CH; j++)
+    if (j < S) cur[j] = xi.raw(xo + (long)j * P);
+  if (t < S) {
+    const double2 tr = a.tau[inst * S + t];
+    tq[t] = (tr.x + tr.y * (double)step_ctr[1]) / a.dslip[t];
+  }
+  const bool project = OPT && o.project;
+  if (!project) {
+    fft_pencils<T, N, 1>(g, l, l, pen, 1 << 30, K::NPEN, fq, (T)1, twl, [&] { ts.store(twl); });
+  } else {
+    ts.store(twl);
+    __syncthreads();
+  }
+  cx<T>* cell = sm + (t / N) * (R * LD) + lds_pos<SH>(t % N);
+  cx<T> r[R];
+  double2 s[R];
+#pragma unroll
+  for (int c = 0; c < R; c++) {
+    r[c] = cell[c * LD];
+    s[c] = make_double2(0.0, 0.0);
+  }
+#pragma unroll 1
+  for (int a0 = 0; a0 < S; a0 += CH) {
+#pragma unroll
+    for (int j = 0; j < CH; j++)
+      if (a0 + CH + j < S) nxt[j] = xi.raw(xo + (long)(a0 + CH + j) * P);
+    double gm[CH];
+#pragma unroll
+    for (int j = 0; j < CH; j++) {
+      gm[j] = 0.0;
+      if (a0 + j >= S) continue;
+      const int f = a0 + j;
+      double2 x = M::widen(cur[j]);
+      if (!project) {
+        double dr = 0.0, di = 0.0;
+#pragma unroll
+        for (int c = 0; c < R; c++) {
+          dr += a.al[f][c] * (double)r[c].x;
+          di += a.al[f][c] * (double)r[c].y;
+        }
+        const long e = xo + (long)f * P;
+        double q = tq[f];
+        bool live = true;
+        if constexpr (OPT) {
+          if (o.extra) {
+            const cx<T> v = o.extra[e];
+            dr += (double)v.x;
+            di += (double)v.y;
+          }
+          if (o.taupp)
+            q = (o.taupp[((long)inst * P + pt0 + t) * S + f] + a.tau[inst * S + f].y * (double)step_ctr[1]) / a.dslip[f];
+          if (o.mask) live = o.mask[e] == 0;
+        }
+        if (live) {
+          gl_point_q<lean_master<M>()>(x, dr, di, a.cd2[f], a.asf_pi[f], q, a);
+          xi.store(e, x);
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < R; c++) {
+        s[c].x += a.al[f][c] * x.x;
+        s[c].y += a.al[f][c] * x.y;
+      }
+      gm[j] = x.x;
+    }
+    const double gs = wave_sum4(gm);
+    if ((t & 63) < CH && a0 + (t & 63) < S) wred[t >> 6][a0 + (t & 63)] = gs;
+#pragma unroll
+    for (int j = 0; j < CH; j++) cur[j] = nxt[j];
+  }
+#pragma unroll
+  for (int c = 0; c < R; c++) cell[c * LD] = {(T)s[c].x, (T)s[c].y};
+  __syncthreads();
+  if (t < S && !project) {
+    double v = 0.0;
+    for (int w = 0; w < NT / 64; w++) v += wred[w][t];
+    partials[((long)inst * S + t) * a.nblk + blk] = v * a.inv_n;
+  }
+  fft_pencils<T, N, 1>(l, l, g, pen, 1 << 30, K::NPEN, fq, (T)-1, twl);
+}
+
+// ---------------------------------------------------------------- column kernel
+// Columns per block TC: row segments (R TC complex) of 128 to 192 bytes where
+// 48 KB of LDS allow it.
+template <typename T, int N, int R> struct ColRed {
+  static constexpr int TPP = make_plan(N).tpp, LD = pitch<N>();
+  static constexpr size_t CSZ = sizeof(cx<T>);
+  static constexpr int tc() {
+    int t = 1;
+    while (t * 2 * R * CSZ <= 192 && (size_t)t * 2 * R * LD * CSZ <= 48 * 1024 && t * 2 * R * TPP <= 1024) t *= 2;
+    return t;
+  }
+  static constexpr int TC = tc(), NPEN = R * TC, LANES = (NPEN * TPP + 63) / 64 * 64;
+  static constexpr int PTS = N * TC < 512 ? N * TC : 512;
+  static constexpr int NT = LANES > PTS ? LANES : (PTS + 63) / 64 * 64;
+};
+
+// The two stages of the per-field sums ride along as extra blocks of the
+// launches that follow the row kernel anyway (as launches of their own they
+// take 5 us each, of the 16 to 25 us that a step of a 32^3 grid takes): when
+// the row kernel wrote many block sums per field, blocks of the forward N2
+// pass fold them to FOLD per field, and one block of the column kernel turns
+// those into the history row.  A field is added by one wave in a fixed order,
+// which is k_finish_sums' order for up to FOLD_ABOVE sums.
+constexpr int FOLD_ABOVE = 512;
+struct FoldJob {
+  const double* in;  // [F][nblk], null: nothing to fold
+  double* out;       // [F][FOLD]
+  int nblk, F;
+};
+struct FinishJob {
+  const double* in;  // [F][nblk], null: the sums are finished elsewhere
+  double* out;       // history
+  int* step_ctr;
+  int nblk, F, S;
+};
+__device__ __forceinline__ double wave_range_sum(const double* __restrict__ v, int b0, int b1) {
+  double acc = 0.0;
+  for (int b = b0 + ((int)threadIdx.x & 63); b < b1; b += 64) acc += v[b];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+  return acc;
+}
+template <int NT> __device__ __forceinline__ void fold_block(const FoldJob& j, int blk) {
+  constexpr int NW = NT / 64;
+  const int w = threadIdx.x >> 6, k = blk * NW + w;
+  if (w >= NW || k >= j.F * FOLD) return;
+  const int f = k / FOLD, part = k % FOLD;
+  const int per = (j.nblk + FOLD - 1) / FOLD, b0 = part * per;
+  const double s = wave_range_sum(j.in + (long)f * j.nblk, b0, b0 + per < j.nblk ? b0 + per : j.nblk);
+  if ((threadIdx.x & 63) == 0) j.out[(long)f * FOLD + part] = s;
+}
+template <int NT> __device__ __forceinline__ void finish_block(const FinishJob& j) {
+  constexpr int NW = NT / 64;
+  const int ninst = j.F / j.S;
+  double* dst = j.out + (long)j.step_ctr[0] * ninst * (j.S + 1);
+  for (int f = threadIdx.x >> 6; f < j.F; f += NW) {
+    const double s = wave_range_sum(j.in + (long)f * j.nblk, 0, j.nblk);
+    if ((threadIdx.x & 63) == 0) dst[(f / j.S) * (j.S + 1) + f % j.S] = s;
+  }
+  __syncthreads();
+  for (int b = threadIdx.x; b < ninst; b += NT) {
+    double tot = 0.0;
+    for (int a = 0; a < j.S; a++) tot += dst[b * (j.S + 1) + a];
+    dst[b * (j.S + 1) + j.S] = tot;
+  }
+  if (threadIdx.x == 0) {
+    j.step_ctr[0] = j.step_ctr[0] + 1;  // history row (read by every thread before the barrier above)
+    j.step_ctr[1] = j.step_ctr[1] + 1;  // GL steps since the tau ramp was set
+  }
+}
+
+// Stored mode: K(k) as its upper triangle in the working precision, the
+// R (R + 1) / 2 values of a k-point together (so that a column tile reads them
+// in stretches, as it reads W), built once in FP64.  One thread per k-point.
+constexpr int red_tri(int a, int b, int R) { return a * R - a * (a - 1) / 2 + (b - a); }  // a <= b
+template <typename T, int R>
+__global__ void __launch_bounds__(256)
+k_build_K(T* __restrict__ Kst, const ElasticConsts* __restrict__ ec, long P) {
+  const long pt = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (pt >= P) return;
+  double f[3], g[6], u[R][3];
+  kvec(pt, ec, f);
+  const bool nz = green6(f, ec, g);
+#pragma unroll
+  for (int b = 0; b < R; b++) sig_f(ec, b, f, u[b]);
+#pragma unroll
+  for (int a = 0; a < R; a++) {
+    double gu[3];
+    gmul(g, u[a], gu);
+#pragma unroll
+    for (int b = a; b < R; b++)
+      Kst[pt * (R * (R + 1) / 2) + red_tri(a, b, R)] =
+          nz ? (T)((ec->SE[a][b] - (gu[0] * u[b][0] + gu[1] * u[b][1] + gu[2] * u[b][2])) * ec->inv_mu) : (T)0;
+  }
+}
+template <typename T, int R>
+__device__ __forceinline__ void contract_stored_lds(cx<T>* io, int stride, const T* __restrict__ k) {
+  T kv[R * (R + 1) / 2];
+#pragma unroll
+  for (int i = 0; i < R * (R + 1) / 2; i++) kv[i] = k[i];
+  cx<T> v[R];
+#pragma unroll
+  for (int b = 0; b < R; b++) v[b] = io[b * stride];
+#pragma unroll
+  for (int a = 0; a < R; a++) {
+    cx<T> o = {(T)0, (T)0};
+#pragma unroll
+    for (int b = 0; b < R; b++) {
+      const T w = kv[a <= b ? red_tri(a, b, R) : red_tri(b, a, R)];
+      o.x += w * v[b].x;
+      o.y += w * v[b].y;
+    }
+    io[a * stride] = o;
+  }
+}
+
+// One block: TC neighbouring (i2, i3) columns of all R components.  Forward
+// N1 transform (last pass of G.c:4599), the contraction K(k) at every k of
+// the columns (G.c:4609-4629 in the basis h_t; ec holds the basis strains in
+// the place of the eigenstrains), inverse N1 transform (first pass of
+// G.c:4638).  grid = instances x column tiles, and one block for the sums.
+template <typename T, int N, int R, bool STORED>
+__global__ void __launch_bounds__((ColRed<T, N, R>::NT))
+k_col_red(cx<T>* __restrict__ W, const ElasticConsts* __restrict__ ec, const T* __restrict__ Kst, long P, int blocks,
+          const cx<T>* __restrict__ tw, const FinishJob fin) {
+  using K = ColRed<T, N, R>;
+  constexpr int NT = K::NT, LD = K::LD, TPP = K::TPP, TC = K::TC, NPEN = K::NPEN;
+  __shared__ cx<T> sm[NPEN * LD];
+  __shared__ cx<T> twl[N];
+  if ((int)blockIdx.x >= blocks) {
+    finish_block<NT>(fin);
+    return;
+  }
+  const int t = threadIdx.x;
+  const long cols = P / N, tiles = cols / TC;
+  const long bt = xcd_tile(blockIdx.x, blocks), inst = bt / tiles, m0 = (bt - inst * tiles) * TC;
+  const int fp = t % NPEN, fq = t / NPEN;
+  const int pen = fq < TPP ? fp : 1 << 30;
+  const StridedPencil<T> g{W + (inst * P + m0) * R + fp, cols * R};
+  const LdsPencils<T> l{sm, LD};
+  TwStage<T, N, NT> ts;
+  ts.load(tw);
+  fft_pencils<T, N, 1>(g, l, l, pen, 1 << 30, NPEN, fq, (T)-1, twl, [&] { ts.store(twl); });
+  for (int e = t; e < N * TC; e += NT) {
+    const int c = e / N, n = e % N;
+    const long pt = (long)n * cols + m0 + c;
+    if constexpr (STORED) contract_stored_lds<T, R>(sm + c * (R * LD) + n, LD, Kst + pt * (R * (R + 1) / 2));
+    else contract_stress_form_lds<T, R>(sm + c * (R * LD) + n, LD, ec, pt);
+  }
+  __syncthreads();
+  fft_pencils<T, N, 1>(l, l, g, pen, 1 << 30, NPEN, fq, (T)1, twl);
+}
+
+// ---------------------------------------------------------------- N2 pass
+// Transform along N2 of the [outer][N][inner] components (inner = N3 R), as
+// k_fft_cols; the last tile of a row may be narrower than the others.
+// grid = fold blocks, then outer x tiles.
+template <typename T, int N>
+__global__ void __launch_bounds__((cols_threads<T, N>()))
+k_pass2_red(cx<T>* __restrict__ data, int inner, int blocks, T sign, const cx<T>* __restrict__ tw, const FoldJob fold,
+            int nfold) {
+  constexpr int TILE = tile_cols<T, N>(), LD = pitch<N>(), NT = cols_threads<T, N>();
+  extern __shared__ unsigned char lds_raw[];  // cols_lds_bytes<T, N>()
+  cx<T>* sm = reinterpret_cast<cx<T>*>(lds_raw);
+  __shared__ cx<T> twl[N];
+  if ((int)blockIdx.x < nfold) {
+    fold_block<NT>(fold, blockIdx.x);
+    return;
+  }
+  TwStage<T, N, NT> ts;
+  ts.load(tw);
+  const int tiles = (inner + TILE - 1) / TILE;
+  const long bt = xcd_tile((int)blockIdx.x - nfold, blocks);
+  const long o = bt / tiles;
+  const int i0 = (int)(bt - o * tiles) * TILE, np = inner - i0 < TILE ? inner - i0 : TILE;
+  const ColPencils<T> g{data + o * N * inner + i0, inner};
+  const LdsPencils<T> l{sm, LD};
+  fft_pencils<T, N, 1>(g, l, g, (int)threadIdx.x % TILE, 1 << 30, np, (int)threadIdx.x / TILE, sign, twl,
+                       [&] { ts.store(twl); });
+}
+
+}  // namespace pfdd

@@ -1,0 +1,132 @@
+"""GPU parity of the reduced-basis GL step (AUTO on grids whose N1 and N3 have
+fused kernels): against the FP64 oracle and against the field-major kernels,
+for every number of components, at every fused length of either axis, with
+each option of the update.
+
+Tolerances: FP64 as in the other parity tests (1e-12 against the oracle after
+12 steps); the FP32 modes differ from their field-major runs by the FP32
+rounding of the transforms (a few 2^-24 of values of order 1 a step): 2e-6."""
+import sys
+
+import numpy as np
+import pytest
+
+import oraclepy as O
+import pfdd_amd as pa
+from pfdd_amd import configs as C
+from pfdd_amd import hip
+
+pytestmark = pytest.mark.gpu
+PRECS = [pa.FP64, pa.MIXED, pa.MIXED_LEAN]
+FUSED = (32, 48, 64, 96, 128, 192, 256, 384, 512)
+
+
+@pytest.fixture(scope="module", autouse=True)
+def need_gpu():
+    if hip.device_count() < 1:
+        pytest.skip("no GPU visible")
+
+
+def options(w, masked, tau_pp):
+    rng = np.random.default_rng(17)
+    bc = None
+    if masked:
+        bc = (rng.random((w.ns,) + w.shape) < 0.1).astype(np.complex128)
+    tau = rng.uniform(-0.02, 0.02, (w.P, w.ns)) if tau_pp else w.tau
+    return bc, tau
+
+
+def gpu(w, plan, prec, steps=12, bc=None, tau=None, quirk=True, bmode=pa.B_RECOMPUTE, eps=None, chunks=()):
+    p = w.params(prec, bmode, plan)
+    with pa.Context(p) as c:
+        c.set_tau(w.tau if tau is None else tau, per_point=tau is not None and np.ndim(tau) == 2)
+        c.upload_xi(w.xi, bc)
+        c.begin_outer(quirk)
+        out = [c.gl_steps(n)[1] for n in (chunks or (steps,))]
+        return c.download_xi(), np.concatenate(out)
+
+
+def oracle(w, steps=12, bc=None, tau=None, quirk=True):
+    o = O.Oracle(O.make_params(w.shape, w.eps, C.C11, C.C12, C.C44, [0.1] * w.ns, C.asf2_reference(w.ns),
+                               [1.0] * w.ns))
+    o.set_xi(w.xi, bc)
+    o.set_tau(w.tau if tau is None else tau, per_point=tau is not None and np.ndim(tau) == 2)
+    o.prologue(quirk)
+    _, ga = o.gl_steps(steps)
+    x = o.get_xi()
+    o.close()
+    return x, ga
+
+
+def check(w, prec, bc=None, tau=None, quirk=True, bmode=pa.B_RECOMPUTE):
+    tau_arg = tau if tau is not None and np.ndim(tau) == 2 else None
+    x1, g1 = gpu(w, pa.PLAN_AUTO, prec, bc=bc, tau=tau_arg, quirk=quirk, bmode=bmode)
+    if prec == pa.FP64:
+        xo, go = oracle(w, bc=bc, tau=tau_arg, quirk=quirk)
+        assert np.abs(x1 - xo).max() <= 1e-12
+        assert np.abs(g1 - go).max() <= 1e-12
+    else:
+        x0, g0 = gpu(w, pa.PLAN_FIELD_MAJOR | pa.PLAN_NO_PLANE, prec, bc=bc, tau=tau_arg, quirk=quirk, bmode=bmode)
+        assert np.abs(x1 - x0).max() <= 2e-6
+        assert np.abs(g1 - g0).max() <= 2e-6
+
+
+@pytest.mark.parametrize("prec", PRECS)
+@pytest.mark.parametrize("ns", range(1, 13))
+def test_component_counts(ns, prec):
+    """ns = 1..12 of the FCC systems: 1, 2, 2, 3, 4, 4, 5 ... 5 components."""
+    check(C.small_fcc((32, 4, 32), ns=ns), prec)
+
+
+def test_six_components():
+    """Strains with a trace (no slip systems) span all six dimensions."""
+    w = C.small_fcc((32, 2, 32), ns=7)
+    rng = np.random.default_rng(3)
+    w.eps = w.eps + 0.3 * rng.standard_normal(w.eps.shape)
+    check(w, pa.FP64)
+
+
+@pytest.mark.parametrize("prec", PRECS)
+@pytest.mark.parametrize("n", FUSED)
+def test_lengths_of_the_row_and_column_kernels(n, prec):
+    """Each length along N1 and along N3, five components and two; N2 = 3 and 6."""
+    for shape, ns in (((n, 3, 32), 12), ((32, 6, n), 12), ((n, 2, 48), 3), ((48, 3, n), 3)):
+        check(C.small_fcc(shape, ns=ns, nloops=3), prec)
+
+
+@pytest.mark.parametrize("prec", PRECS)
+@pytest.mark.parametrize("masked,tau_pp", [(True, False), (False, True), (True, True)])
+def test_frozen_points_and_per_point_shear(masked, tau_pp, prec):
+    w = C.small_fcc((48, 6, 64), ns=5)
+    bc, tau = options(w, masked, tau_pp)
+    check(w, prec, bc=bc, tau=tau)
+    if masked:
+        x, _ = gpu(w, pa.PLAN_AUTO, pa.FP64, bc=bc)
+        assert np.array_equal(x[bc != 0], w.xi[bc != 0])
+
+
+@pytest.mark.parametrize("quirk", [True, False])
+def test_prologue_term_and_first_step(quirk):
+    """The prologue's per-field term enters the first update only, however the
+    steps are split over calls (eager first step, graph replays, eager rest)."""
+    w = C.small_fcc((32, 8, 32), ns=6)
+    check(w, pa.FP64, quirk=quirk)
+    x1, g1 = gpu(w, pa.PLAN_AUTO, pa.FP64, quirk=quirk, chunks=(21,))
+    x2, g2 = gpu(w, pa.PLAN_AUTO, pa.FP64, quirk=quirk, chunks=(1, 8, 9, 3))
+    assert np.array_equal(x1, x2) and np.array_equal(g1, g2)
+
+
+@pytest.mark.parametrize("prec", PRECS)
+def test_ensemble_class_equals_single(prec):
+    """Instances of a batched class get the bits of their own contexts."""
+    members = [C.small_fcc((32, 4, 48), ns=3, seed=C.BASE_SEED + 500 + i) for i in range(3)]
+    with pa.Ensemble([m.params(prec) for m in members]) as e:
+        for i, m in enumerate(members):
+            e.set_tau(i, m.tau)
+            e.upload_xi(i, m.xi)
+        e.begin_outer(True)
+        g = e.gl_steps(19)
+        for i, m in enumerate(members):
+            x, ga = gpu(m, pa.PLAN_AUTO, prec, steps=19)
+            assert np.array_equal(e.download_xi(i), x)
+            assert np.abs(g[:, i] - ga.sum(1)).max() <= 1e-14
