@@ -40,13 +40,14 @@ def _run(cmd):
 
 
 def _fresh(obj, src):
-    """obj exists and is newer than src and every header it may include."""
-    if not os.path.exists(obj):
+    """obj exists and is newer than src and the headers its dependency file names."""
+    dep = obj + ".d"
+    if not os.path.exists(obj) or not os.path.exists(dep):
         return False
-    deps = [src] + [os.path.join(CSRC, h) for h in os.listdir(CSRC) if h.endswith((".hpp", ".h"))] + \
-        [os.path.join(INC, h) for h in os.listdir(INC)]
+    with open(dep) as fh:
+        names = [n for n in fh.read().replace("\\\n", " ").split() if not n.endswith(":") and n.startswith(ROOT)]
     t = os.path.getmtime(obj)
-    return all(os.path.getmtime(d) < t for d in deps)
+    return all(os.path.exists(d) and os.path.getmtime(d) < t for d in names + [src])
 
 
 def build(verbose=False, incremental=False):
@@ -57,13 +58,14 @@ def build(verbose=False, incremental=False):
         objs.append(o)
         if incremental and _fresh(o, os.path.join(CSRC, s)):
             continue
-        _run(["gcc", "-O2", "-fPIC", "-std=c99", "-Wall", f"-I{INC}", "-c", os.path.join(CSRC, s), "-o", o])
+        _run(["gcc", "-O2", "-fPIC", "-std=c99", "-Wall", f"-I{INC}", "-MMD", "-MF", o + ".d", "-c",
+              os.path.join(CSRC, s), "-o", o])
 
     def compile_unit(unit):
         src, obj, flags = unit
         o = os.path.join(BUILD, obj)
         if not (incremental and _fresh(o, os.path.join(CSRC, src))):
-            out = _run([HIPCC] + HIP_FLAGS + flags + ["-c", os.path.join(CSRC, src), "-o", o])
+            out = _run([HIPCC] + HIP_FLAGS + flags + ["-MMD", "-MF", o + ".d", "-c", os.path.join(CSRC, src), "-o", o])
             if verbose and out.strip():
                 print(out)
         return o

@@ -1280,11 +1280,10 @@ int build_stored(pfdd_ctx* c) {
   return hipPeekAtLastError() == hipSuccess ? PFDD_OK : PFDD_E_HIP;
 }
 
-// Whether AUTO runs the steps in the reduced basis: wherever the fused row
-// and column lengths exist.
+// Whether AUTO runs the steps in the reduced basis.
 bool auto_reduced(const pfdd_ctx* c, int plan) {
   const pfdd_params& p = c->p;
-  if (plan != PFDD_PLAN_AUTO || !fused_len(p.n1) || !fused_len(p.n3)) return false;
+  if (plan != PFDD_PLAN_AUTO) return false;
   const size_t csz = c->fp64 ? sizeof(double2) : sizeof(float2);
   if (!c->stored && p.n1 == p.n3 && il_fixed_S(p.n1) == c->S && csz * c->S * c->P <= (128u << 20)) return false;
   return true;
@@ -1355,7 +1354,8 @@ int apply_plan(pfdd_ctx* c, int plan) {
     c->row_tile = c->c3_tile = 0;
     c->c3_lds = 0;
     c->plane = c->il = c->il_fixed = c->il_fixed_row = 0;
-    c->row_nblk = p.n1 * p.n2 / red_rows(p.n3);
+    const int rows = red_row_rows(c->fp64 != 0, p.n3, c->red_R, S);
+    c->row_nblk = (p.n1 * p.n2 + rows - 1) / rows;
     c->red = 1;
     drop_graph(c);
     c->plan = plan;

@@ -1,10 +1,62 @@
-// pfdd_reduced.h -- launchers of the reduced-basis kernels (pfdd_reduced.hip,
-// compiled once per component count R and kind so that the instantiations
-// build in parallel).
+// pfdd_reduced.h -- arguments and launchers of the reduced-basis kernels
+// (pfdd_reduced.hpp holds the kernels and says what they compute;
+// pfdd_reduced.hip is compiled once per component count R and kind so that the
+// instantiations build in parallel).
 #pragma once
-#include "pfdd_reduced.hpp"
+#include "pfdd_kernels.hpp"
 
 namespace pfdd {
+
+constexpr int RED_MAXR = 6;
+
+// What the row kernel needs of the step (by value, read through the scalar cache).
+struct RedArgs {
+  long P;
+  int S;
+  int nblk;                    // row blocks per field
+  double uq2, two_pi, inv_n;
+  double cd2[MAXS], asf_pi[MAXS], dslip[MAXS];
+  double al[MAXS][RED_MAXR];   // e_a = sum_t al[a][t] h_t
+  const double2* tau;          // per field: (tau, rate)
+};
+// Options of the general variant (OPT): frozen points, per-point shear, the
+// prologue's extra force (virtualevolv G.c:1426-1447, per field in real
+// space), and the projection alone (the prologue: no inverse transform, no
+// update).  Null pointers switch the first three off.
+template <typename T> struct RedOpt {
+  const uint8_t* mask;
+  const double* taupp;
+  const cx<T>* extra;
+  int project;
+};
+
+// Shapes of the row kernels (see there).
+constexpr int red_unrolled(int R) { return R <= 3 ? 4 : R == 4 ? 8 : 0; }  // most fields of k_row_red
+constexpr int red_ppt(bool fp64, int n, int R) { return n <= 64 || R > 3 ? 1 : fp64 || R == 3 ? 2 : 4; }
+constexpr int red_rows(int n, int ppt) {
+  if (n < 32) return 128 / n;
+  const int pts = n % 3 == 0 ? 192 * ppt : ppt == 4 ? 512 : 256;  // points per block
+  return n <= 64 ? 4 : pts / n > 0 ? pts / n : 1;
+}
+// rows per block for ns fields in R components
+constexpr int red_row_rows(bool fp64, int n, int R, int ns) {
+  return red_rows(n, ns <= red_unrolled(R) ? red_ppt(fp64, n, R) : 1);
+}
+
+// The per-field sums that ride along with the N2 pass and the column kernel.
+constexpr int FOLD_ABOVE = 512;
+struct FoldJob {
+  const double* in;  // [F][nblk], null: nothing to fold
+  double* out;       // [F][FOLD]
+  int nblk, F;
+};
+struct FinishJob {
+  const double* in;  // [F][nblk], null: the sums are finished elsewhere
+  double* out;       // history
+  int* step_ctr;
+  int nblk, F, S;
+};
+
 
 template <typename T> struct RedRowLaunch {
   RedArgs a;

@@ -1,7 +1,7 @@
 // pfdd_reduced.hip -- instantiations of the reduced-basis kernels.  Compiled
 // with -DPFDD_RED_R=1..6 and -DPFDD_RED_KIND=0..3 (row kernel on the FP64,
 // compensated or lean master; column kernels), and once with KIND 4 (N2 pass).
-#include "pfdd_reduced.h"
+#include "pfdd_reduced.hpp"
 
 namespace pfdd {
 namespace {
@@ -12,17 +12,32 @@ constexpr int R = PFDD_RED_R;
 
 #if PFDD_RED_KIND < 3
 template <typename T, int N, typename M> void row(const RedRowLaunch<T>& q, M xi) {
-  const dim3 grid(q.nblk, q.batch), block(RowRed<T, N, R>::NT);
-  if (q.o.mask || q.o.taupp || q.o.extra || q.o.project)
-    hipLaunchKernelGGL((k_row_red<T, N, R, M, true>), grid, block, 0, q.stream, q.W, xi, q.a, q.o, q.tw, q.partials,
+  const dim3 grid(q.nblk, q.batch);
+  const bool opt = q.o.mask || q.o.taupp || q.o.extra || q.o.project;
+  if constexpr (red_unrolled(R) > 0) {
+    if (q.a.S <= red_unrolled(R)) {
+      const dim3 block(RowRed<T, N, R, red_ppt(sizeof(T) == 8, N, R)>::NT);
+      if (opt)
+        hipLaunchKernelGGL((k_row_red<T, N, R, M, true>), grid, block, 0, q.stream, q.W, xi, q.a, q.o, q.tw, q.partials,
+                           q.step_ctr);
+      else
+        hipLaunchKernelGGL((k_row_red<T, N, R, M, false>), grid, block, 0, q.stream, q.W, xi, q.a, q.o, q.tw,
+                           q.partials, q.step_ctr);
+      return;
+    }
+  }
+  const dim3 block(RowRed<T, N, R, 1>::NT);
+  if (opt)
+    hipLaunchKernelGGL((k_row_red_n<T, N, R, M, true>), grid, block, 0, q.stream, q.W, xi, q.a, q.o, q.tw, q.partials,
                        q.step_ctr);
   else
-    hipLaunchKernelGGL((k_row_red<T, N, R, M, false>), grid, block, 0, q.stream, q.W, xi, q.a, q.o, q.tw, q.partials,
+    hipLaunchKernelGGL((k_row_red_n<T, N, R, M, false>), grid, block, 0, q.stream, q.W, xi, q.a, q.o, q.tw, q.partials,
                        q.step_ctr);
 }
 template <typename T, typename M> bool row_any(const RedRowLaunch<T>& q, M xi, int n3) {
   switch (n3) {
 #define PFDD_L(NN) case NN: row<T, NN>(q, xi); return true;
+    PFDD_L(2) PFDD_L(3) PFDD_L(4) PFDD_L(6) PFDD_L(8) PFDD_L(12) PFDD_L(16) PFDD_L(24)
     PFDD_L(32) PFDD_L(48) PFDD_L(64) PFDD_L(96) PFDD_L(128) PFDD_L(192) PFDD_L(256) PFDD_L(384) PFDD_L(512)
 #undef PFDD_L
     default: return false;
@@ -31,7 +46,7 @@ template <typename T, typename M> bool row_any(const RedRowLaunch<T>& q, M xi, i
 #elif PFDD_RED_KIND == 3
 template <typename T, int N> void col(const RedColLaunch<T>& q) {
   using K = ColRed<T, N, R>;
-  const int blocks = (int)(q.P / N / K::TC * q.batch);
+  const int blocks = (int)((q.P / N + K::TC - 1) / K::TC * q.batch);
   const dim3 grid((unsigned)(blocks + (q.fin.in ? 1 : 0)));
   if (q.Kst)
     hipLaunchKernelGGL((k_col_red<T, N, R, true>), grid, dim3(K::NT), 0, q.stream, q.W, q.ec, q.Kst, q.P, blocks, q.tw,
@@ -46,6 +61,7 @@ template <typename T> void build(T* Kst, const ElasticConsts* ec, long P, hipStr
 template <typename T> bool col_any(const RedColLaunch<T>& q, int n1) {
   switch (n1) {
 #define PFDD_L(NN) case NN: col<T, NN>(q); return true;
+    PFDD_L(2) PFDD_L(3) PFDD_L(4) PFDD_L(6) PFDD_L(8) PFDD_L(12) PFDD_L(16) PFDD_L(24)
     PFDD_L(32) PFDD_L(48) PFDD_L(64) PFDD_L(96) PFDD_L(128) PFDD_L(192) PFDD_L(256) PFDD_L(384) PFDD_L(512)
 #undef PFDD_L
     default: return false;

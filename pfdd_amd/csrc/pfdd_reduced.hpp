@@ -24,32 +24,9 @@
 //
 // Layout: W[instance][N1][N2][N3][R], the components of a point together.
 #pragma once
-#include "pfdd_kernels.hpp"
+#include "pfdd_reduced.h"
 
 namespace pfdd {
-
-constexpr int RED_MAXR = 6;
-
-// What the row kernel needs of the step (by value, read through the scalar cache).
-struct RedArgs {
-  long P;
-  int S;
-  int nblk;                    // row blocks per field
-  double uq2, two_pi, inv_n;
-  double cd2[MAXS], asf_pi[MAXS], dslip[MAXS];
-  double al[MAXS][RED_MAXR];   // e_a = sum_t al[a][t] h_t
-  const double2* tau;          // per field: (tau, rate)
-};
-// Options of the general variant (OPT): frozen points, per-point shear, the
-// prologue's extra force (virtualevolv G.c:1426-1447, per field in real
-// space), and the projection alone (the prologue: no inverse transform, no
-// update).  Null pointers switch the first three off.
-template <typename T> struct RedOpt {
-  const uint8_t* mask;
-  const double* taupp;
-  const cx<T>* extra;
-  int project;
-};
 
 // ---------------------------------------------------------------- wave sums
 template <int CTRL> __device__ __forceinline__ double dpp_mov(double v) {
@@ -58,29 +35,47 @@ template <int CTRL> __device__ __forceinline__ double dpp_mov(double v) {
   const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
-// Sums of four values over a wave at once: lane l with l % 4 = j returns the
-// sum of v[j].  Each of the first two exchanges halves the values a lane
-// carries, so four sums take 33 vector instructions and 4 LDS permutes
-// instead of 4 x 18 and 4 x 4.
-__device__ __forceinline__ double wave_sum4(const double (&v)[4]) {
+// Sums of four values over each row of 16 lanes at once: lane l with
+// l % 4 = j returns the row's sum of v[j].  Each of the first two exchanges
+// halves the values a lane carries, so four sums take 33 vector instructions
+// instead of 4 x 12, and none of them goes through LDS.
+__device__ __forceinline__ double row_sum4(const double (&v)[4]) {
   const bool b0 = threadIdx.x & 1, b1 = threadIdx.x & 2;
-  double k0 = (b0 ? v[1] : v[0]) + dpp_mov<0xB1>(b0 ? v[0] : v[1]);  // quad_perm 1,0,3,2
-  double k1 = (b0 ? v[3] : v[2]) + dpp_mov<0xB1>(b0 ? v[2] : v[3]);
-  double k = (b1 ? k1 : k0) + dpp_mov<0x4E>(b1 ? k0 : k1);           // quad_perm 2,3,0,1
-  k += dpp_mov<0x124>(k);                                            // row_ror 4
-  k += dpp_mov<0x128>(k);                                            // row_ror 8
-  k += __shfl_xor(k, 16, 64);
-  k += __shfl_xor(k, 32, 64);
+  const double k0 = (b0 ? v[1] : v[0]) + dpp_mov<0xB1>(b0 ? v[0] : v[1]);  // quad_perm 1,0,3,2
+  const double k1 = (b0 ? v[3] : v[2]) + dpp_mov<0xB1>(b0 ? v[2] : v[3]);
+  double k = (b1 ? k1 : k0) + dpp_mov<0x4E>(b1 ? k0 : k1);                 // quad_perm 2,3,0,1
+  k += dpp_mov<0x124>(k);                                                  // row_ror 4
+  k += dpp_mov<0x128>(k);                                                  // row_ror 8
   return k;
 }
 
 // ---------------------------------------------------------------- row kernel
-// Rows per block: about 256 points, one per thread.
-constexpr int red_rows(int n) { return n <= 64 ? (n <= 32 ? 4 : n == 48 ? 4 : 4) : n <= 128 ? 2 : 1; }
-template <typename T, int N, int R> struct RowRed {
-  static constexpr int ROWS = red_rows(N), NT = ROWS * N, TPP = make_plan(N).tpp;
+// Two forms of the kernel, by the fields and components:
+//  k_row_red    S <= 4 with R <= 3, and S <= 8 with R = 4: the update is
+//               unrolled over the fields and all master points of a thread
+//               are loaded before the transform, which hides their latency
+//  k_row_red_n  any S: the fields pass through in chunks, the next chunk's
+//               points loaded while one is updated (with 12 fields the first
+//               form needs 146 registers and more in the mixed modes, and
+//               measured 206 against 157 us at 128^3 x 12 mixed)
+// Shape of a block.  The transform occupies R / 8 lanes per point (radix 8),
+// so with one point per thread few lanes of a small R work in it: from N = 96
+// on, R <= 3 takes PPT = 2 points per thread (4 in FP32 with R <= 2); shorter
+// rows keep one, for more blocks on small grids (32^3 x 3: 7 against 9 us).
+// Rows shorter than 32 fill a block of about 128 points with 128 / N of them,
+// and the transform may then need more lanes than there are points.  N1 N2 rows
+// need not be a multiple of ROWS: the last block may be short of rows.
+template <typename T, int N, int R, int PPT_> struct RowRed {
+  static constexpr int PPT = PPT_, ROWS = red_rows(N, PPT), PTS = ROWS * N, TPP = make_plan(N).tpp;
+  static constexpr int LANES = ROWS * R * TPP, NEED = PTS / PPT > LANES ? PTS / PPT : LANES;
+  static constexpr int NT = (NEED + 63) / 64 * 64;
   static constexpr int SH = 3, LD = padded_pitch<N, SH>(), NPEN = ROWS * R;
 };
+// The master advanced by a uniform offset (so that a thread's address is a
+// scalar base and a 32-bit lane offset).
+__device__ __forceinline__ Master<double> advance(Master<double> m, long o) { return {m.p + o}; }
+__device__ __forceinline__ MasterF32C advance(MasterF32C m, long o) { return {m.r + o, m.im + o}; }
+__device__ __forceinline__ MasterF32L advance(MasterF32L m, long o) { return {m.r + o}; }
 
 // A pencil of the interleaved array as one thread sees it: element i at p[i * stride].
 template <typename T> struct StridedPencil {
@@ -90,6 +85,205 @@ template <typename T> struct StridedPencil {
   __device__ __forceinline__ cx<T> load(int, int i) const { return p[i * stride]; }
   __device__ __forceinline__ void store(int, int i, cx<T> v) const { p[i * stride] = v; }
 };
+
+// The update's sine.  Cody-Waite reduction by pi/2 in three parts (the first
+// with 33 bits, so that its products with |k| < 2^20 are exact), the remainder
+// carried as r + t; sin r = r + r^3 S(r^2) and cos r = 1 - r^2/2 + r^4 C(r^2)
+// on |r| <= pi/4 with S and C interpolated at Chebyshev nodes (6 terms each,
+// relative errors 1.3e-17 and 5e-19).  Against 80-bit sinl over 5e6 arguments
+// in each of |x| < 6.3 and |x| < 1000: at most 0.92 ulp, rms 0.295 (correct
+// rounding gives 0.289).  31 vector instructions where the library's sine
+// takes about 60.  Both hold for |x| < SIN_MAX; the row kernel sends larger
+// arguments to big_sin (a function of its own: inlined, the library's long
+// reduction takes 28 registers from the kernel).
+constexpr double SIN_MAX = 4096.0;
+static __device__ __attribute__((noinline, cold)) double big_sin(double x) { return sin(x); }
+// The constants are kept in scalar registers (sgpr_const): left to itself the
+// compiler, in the unrolled update, moves each into a vector register pair at
+// every use, a third of the update's instructions.
+__device__ __forceinline__ double sgpr_const(double v) {
+  asm("" : "+s"(v));
+  return v;
+}
+struct GlSin {
+  const double inv = sgpr_const(0.6366197723675814), p1 = sgpr_const(-1.5707963267341256),
+               p2 = sgpr_const(-6.077100506506192e-11), p3 = sgpr_const(-3.5215598651832e-27),
+               s6 = sgpr_const(1.591805913698281e-10), s5 = sgpr_const(-2.5051130870968297e-08),
+               s4 = sgpr_const(2.755731609787775e-06), s3 = sgpr_const(-0.0001984126983674956),
+               s2 = sgpr_const(0.008333333333330943), s1 = sgpr_const(-0.16666666666666666),
+               c6 = sgpr_const(-1.1382588535352522e-11), c5 = sgpr_const(2.0876145659059344e-09),
+               c4 = sgpr_const(-2.755731726880539e-07), c3 = sgpr_const(2.4801587298760048e-05),
+               c2 = sgpr_const(-0.0013888888888887393), c1 = sgpr_const(0.041666666666666664);
+  __device__ __forceinline__ double operator()(double x) const {
+    const double k = rint(x * inv);
+    const double r1 = fma(k, p1, x), r = fma(k, p2, r1);
+    const double t = fma(k, p3, fma(k, p2, r1 - r));
+    const double z = r * r;
+    double s = fma(z, s6, s5);
+    s = fma(s, z, s4);
+    s = fma(s, z, s3);
+    s = fma(s, z, s2);
+    s = fma(s, z, s1);
+    s = r + fma(r * z, s, t);
+    double c = fma(z, c6, c5);
+    c = fma(c, z, c4);
+    c = fma(c, z, c3);
+    c = fma(c, z, c2);
+    c = fma(c, z, c1);
+    const double w = fma(-0.5, z, 1.0);
+    c = w + fma(z * z, c, fma(-r, t, fma(-0.5, z, 1.0 - w)));
+    const int q = (int)k;
+    const double o = (q & 1) ? c : s;
+    return (q & 2) ? -o : o;
+  }
+};
+// The lean master's sine (xi carries 24 bits): reduction by pi, then 5 terms
+// on |r| <= pi/2, absolute error 7e-11 where an FP32 sine of the reduced
+// argument has 6e-8.
+struct GlSinLean {
+  const double inv = sgpr_const(0.3183098861837907), p1 = sgpr_const(-3.141592653589793),
+               p2 = sgpr_const(-1.2246467991473532e-16), s5 = sgpr_const(-2.4079713707378346e-08),
+               s4 = sgpr_const(2.753644296396837e-06), s3 = sgpr_const(-0.00019841086288980702),
+               s2 = sgpr_const(0.008333332767631813), s1 = sgpr_const(-0.16666666663874308);
+  __device__ __forceinline__ double operator()(double x) const {
+    const double k = rint(x * inv);
+    const double r = fma(k, p2, fma(k, p1, x));
+    const double z = r * r;
+    double s = fma(z, s5, s4);
+    s = fma(s, z, s3);
+    s = fma(s, z, s2);
+    s = fma(s, z, s1);
+    s = fma(r * z, s, r);
+    return ((int)k & 1) ? -s : s;
+  }
+};
+
+// One block: ROWS rows along N3 of all R components.  Inverse N3 transform
+// (G.c:4638), then point by point: the S driving forces from the R components,
+// plasticevolv (G.c:3470-3501) on the S fields, the new components from them,
+// the fields' sums of Re xi / P; forward N3 transform (first pass of
+// G.c:4599).  The first pass reads W into registers and the last writes it
+// back.  A thread's master points are all loaded before the transform, which
+// hides their latency.  Bound by HBM at R = 2 and 3 (256x256x192 x 3: FP64
+// 322 us, 6.25 TB/s; mixed 214 us, 6.1 TB/s), with one point per thread and the
+// points loaded a chunk ahead 395 and 377 us.  S <= SM.  grid = (row blocks,
+// instances).
+template <typename T, int N, int R, typename M, bool OPT>
+__global__ void __launch_bounds__((RowRed<T, N, R, red_ppt(sizeof(T) == 8, N, R)>::NT), N == 512 ? 1 : 4)
+k_row_red(cx<T>* __restrict__ W, M xi, const RedArgs a, const RedOpt<T> o, const cx<T>* __restrict__ tw,
+          double* __restrict__ partials, const int* __restrict__ step_ctr) {
+  using K = RowRed<T, N, R, red_ppt(sizeof(T) == 8, N, R)>;
+  constexpr int NT = K::NT, LD = K::LD, TPP = K::TPP, SH = K::SH, ROWS = K::ROWS, PPT = K::PPT, SM = red_unrolled(R);
+  static_assert(K::LANES <= NT && SM % 4 == 0 && NT >= MAXS, "block shape");
+  __shared__ cx<T> sm[K::NPEN * LD];
+  __shared__ cx<T> twl[N];
+  __shared__ double tq[MAXS], rowsum[NT / 16][MAXS];
+  const int t = threadIdx.x, S = a.S, inst = blockIdx.y;
+  const long blk = blockIdx.x, P = a.P, pt0 = blk * (ROWS * N);
+  // FFT lanes: component fastest, then the lane within the pencil, then the row
+  const int fc = t % R, fq = (t / R) % TPP, fr = t / (R * TPP);
+  const int nr = P / N - blk * ROWS < ROWS ? (int)(P / N - blk * ROWS) : ROWS;  // rows of this block
+  const int pen = fr < nr ? fr * R + fc : 1 << 30;
+  const StridedPencil<T> g{W + ((long)inst * P + pt0 + (long)fr * N) * R + fc, R};
+  const LdsPencils<T, SH> l{sm, LD};
+  TwStage<T, N, NT> ts;
+  ts.load(tw);
+  const long x0 = (long)inst * S * P + pt0;  // the block's first point of field 0
+  typename M::Raw raw[PPT][SM];
+#pragma unroll
+  for (int f = 0; f < SM; f++)
+    if (f < S) {
+      const M m = advance(xi, x0 + (long)f * P);
+#pragma unroll
+      for (int p = 0; p < PPT; p++)  // (a lane without a point loads the block's first)
+        raw[p][f] = m.raw(t + p * NT < nr * N ? t + p * NT : 0);
+    }
+  if (t < S) {
+    const double2 tr = a.tau[inst * S + t];
+    tq[t] = (tr.x + tr.y * (double)step_ctr[1]) / a.dslip[t];
+  }
+  const bool project = OPT && o.project;
+  if (!project) {
+    fft_pencils<T, N, 1>(g, l, l, pen, 1 << 30, K::NPEN, fq, (T)1, twl, [&] { ts.store(twl); });
+  } else {
+    ts.store(twl);
+    __syncthreads();
+  }
+  const std::conditional_t<lean_master<M>(), GlSinLean, GlSin> glsin;
+  double gsum[SM];
+#pragma unroll
+  for (int f = 0; f < SM; f++) gsum[f] = 0.0;
+#pragma unroll
+  for (int p = 0; p < PPT; p++) {
+    const int e0 = t + p * NT;  // the point within the block
+    if (e0 >= nr * N) continue;
+    cx<T>* cell = sm + (e0 / N) * (R * LD) + lds_pos<SH>(e0 % N);
+    double2 r[R], s[R];
+#pragma unroll
+    for (int c = 0; c < R; c++) {
+      const cx<T> v = cell[c * LD];
+      r[c] = make_double2((double)v.x, (double)v.y);
+      s[c] = make_double2(0.0, 0.0);
+    }
+#pragma unroll
+    for (int f = 0; f < SM; f++) {
+      if (f >= S) continue;
+      double2 x = M::widen(raw[p][f]);
+      if (!project) {
+        double dr = 0.0, di = 0.0;
+#pragma unroll
+        for (int c = 0; c < R; c++) {
+          dr += a.al[f][c] * r[c].x;
+          di += a.al[f][c] * r[c].y;
+        }
+        double q = tq[f];
+        bool live = true;
+        if constexpr (OPT) {
+          const long e = x0 + (long)f * P + e0;
+          if (o.extra) {
+            const cx<T> v = o.extra[e];
+            dr += (double)v.x;
+            di += (double)v.y;
+          }
+          if (o.taupp)
+            q = (o.taupp[((long)inst * P + pt0 + e0) * S + f] + a.tau[inst * S + f].y * (double)step_ctr[1]) /
+                a.dslip[f];
+          if (o.mask) live = o.mask[e] == 0;
+        }
+        if (live) {
+          const double arg = a.two_pi * x.x;
+          double sn = glsin(arg);
+          if (__builtin_expect(fabs(arg) > SIN_MAX, 0)) sn = big_sin(arg);
+          x.x -= a.cd2[f] * (a.uq2 * dr * a.inv_n + a.asf_pi[f] * sn - q);  // G.c:3485-3489
+          x.y -= a.uq2 * a.cd2[f] * (di * a.inv_n);
+          advance(xi, x0 + (long)f * P).store(e0, x);
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < R; c++) {
+        s[c].x += a.al[f][c] * x.x;
+        s[c].y += a.al[f][c] * x.y;
+      }
+      gsum[f] += x.x;
+    }
+#pragma unroll
+    for (int c = 0; c < R; c++) cell[c * LD] = {(T)s[c].x, (T)s[c].y};
+  }
+#pragma unroll
+  for (int f = 0; f < SM; f += 4) {
+    if (f >= S) continue;
+    const double v[4] = {gsum[f], gsum[f + 1], gsum[f + 2], gsum[f + 3]};
+    const double rs = row_sum4(v);
+    if ((t & 15) < 4) rowsum[t >> 4][f + (t & 15)] = rs;
+  }
+  __syncthreads();
+  if (t < S && !project) {
+    double v = 0.0;
+    for (int w = 0; w < NT / 16; w++) v += rowsum[w][t];
+    partials[((long)inst * S + t) * a.nblk + blk] = v * a.inv_n;
+  }
+  fft_pencils<T, N, 1>(l, l, g, pen, 1 << 30, K::NPEN, fq, (T)-1, twl);
+}
 
 // plasticevolv (G.c:3485-3489) with the shear already divided by dslip.
 template <bool F32SIN>
@@ -108,32 +302,38 @@ __device__ __forceinline__ void gl_point_q(double2& x, double dre, double dim, d
   x.y -= a.uq2 * cd2 * (dim * a.inv_n);
 }
 
-// One block: ROWS rows along N3 of all R components.  Inverse N3 transform
-// (G.c:4638), then one point per thread: the S driving forces from the R
-// components, plasticevolv (G.c:3470-3501) on the S fields of the point, the
-// new components from them, the fields' sums of Re xi / P; forward N3
-// transform (first pass of G.c:4599).  The first pass reads W into registers
-// and the last writes it back.  grid = (row blocks, instances).
+// The form for any S.  Chunk length and register bound by measurement, at
+// 128^3 x 12 and 256x256x128 x 12 (us): FP64 chunks of 4 without a bound 183
+// and 786 (chunks of 2 with four waves a SIMD 177 and 820); the compensated
+// mode chunks of 2 and four waves 155 and 559 (chunks of 4: 155 and 572); lean
+// chunks of 4 and five waves 106 (115 without the bound).  FP64 runs at HBM
+// speed (6.3 TB/s); the mixed modes are bound by vector issue (69% of the
+// cycles).  Its sine is the library's: with GlSin it measured slower in FP64
+// and lean (187 and 115 us), where the constants crowd out points in flight.
+template <typename M> constexpr int row_n_chunk() { return __is_same(M, MasterF32C) ? 2 : 4; }
+template <typename M> constexpr int row_n_waves() { return __is_same(M, MasterF32C) ? 4 : lean_master<M>() ? 5 : 1; }
 template <typename T, int N, int R, typename M, bool OPT>
-__global__ void __launch_bounds__((RowRed<T, N, R>::NT))
-k_row_red(cx<T>* __restrict__ W, M xi, const RedArgs a, const RedOpt<T> o, const cx<T>* __restrict__ tw,
+__global__ void __launch_bounds__((RowRed<T, N, R, 1>::NT), (row_n_waves<M>()))
+k_row_red_n(cx<T>* __restrict__ W, M xi, const RedArgs a, const RedOpt<T> o, const cx<T>* __restrict__ tw,
           double* __restrict__ partials, const int* __restrict__ step_ctr) {
-  using K = RowRed<T, N, R>;
-  constexpr int NT = K::NT, LD = K::LD, TPP = K::TPP, SH = K::SH, ROWS = K::ROWS, CH = 4;
-  static_assert(NT % 64 == 0 && R * TPP <= N, "one pencil per lane group");
+  using K = RowRed<T, N, R, 1>;
+  constexpr int NT = K::NT, LD = K::LD, TPP = K::TPP, SH = K::SH, ROWS = K::ROWS, CH = row_n_chunk<M>();
+  static_assert(K::LANES <= NT && NT >= MAXS, "block shape");
   __shared__ cx<T> sm[K::NPEN * LD];
   __shared__ cx<T> twl[N];
-  __shared__ double tq[MAXS], wred[NT / 64][MAXS];
+  __shared__ double tq[MAXS], rowsum[NT / 16][MAXS];
   const int t = threadIdx.x, S = a.S, inst = blockIdx.y;
-  const long blk = blockIdx.x, P = a.P, pt0 = blk * NT;
+  const long blk = blockIdx.x, P = a.P, pt0 = blk * (ROWS * N);  // one point per thread
   // FFT lanes: component fastest, then the lane within the pencil, then the row
   const int fc = t % R, fq = (t / R) % TPP, fr = t / (R * TPP);
-  const int pen = fr < ROWS ? fr * R + fc : 1 << 30;
+  const int nr = P / N - blk * ROWS < ROWS ? (int)(P / N - blk * ROWS) : ROWS;  // rows of this block
+  const int pen = fr < nr ? fr * R + fc : 1 << 30;
   const StridedPencil<T> g{W + ((long)inst * P + pt0 + (long)fr * N) * R + fc, R};
   const LdsPencils<T, SH> l{sm, LD};
   TwStage<T, N, NT> ts;
   ts.load(tw);
-  const long xo = (long)inst * S * P + pt0 + t;  // this thread's point of field 0
+  const long xo = (long)inst * S * P + pt0 + (t < nr * N ? t : 0);  // this thread's point of field 0 (or the block's first)
+  const bool has = t < nr * N;  // this thread has a point
   typename M::Raw cur[CH], nxt[CH];
 #pragma unroll
   for (int j = 0; j < CH; j++)
@@ -149,7 +349,7 @@ k_row_red(cx<T>* __restrict__ W, M xi, const RedArgs a, const RedOpt<T> o, const
     ts.store(twl);
     __syncthreads();
   }
-  cx<T>* cell = sm + (t / N) * (R * LD) + lds_pos<SH>(t % N);
+  cx<T>* cell = sm + (has ? (t / N) * (R * LD) + lds_pos<SH>(t % N) : 0);
   cx<T> r[R];
   double2 s[R];
 #pragma unroll
@@ -166,7 +366,7 @@ k_row_red(cx<T>* __restrict__ W, M xi, const RedArgs a, const RedOpt<T> o, const
 #pragma unroll
     for (int j = 0; j < CH; j++) {
       gm[j] = 0.0;
-      if (a0 + j >= S) continue;
+      if (a0 + j >= S || !has) continue;
       const int f = a0 + j;
       double2 x = M::widen(cur[j]);
       if (!project) {
@@ -201,17 +401,21 @@ k_row_red(cx<T>* __restrict__ W, M xi, const RedArgs a, const RedOpt<T> o, const
       }
       gm[j] = x.x;
     }
-    const double gs = wave_sum4(gm);
-    if ((t & 63) < CH && a0 + (t & 63) < S) wred[t >> 6][a0 + (t & 63)] = gs;
+    double v4[4] = {gm[0], gm[1], 0.0, 0.0};
+    if constexpr (CH == 4) v4[2] = gm[2], v4[3] = gm[3];
+    const double rs = row_sum4(v4);
+    if ((t & 15) < CH) rowsum[t >> 4][a0 + (t & 15)] = rs;
 #pragma unroll
     for (int j = 0; j < CH; j++) cur[j] = nxt[j];
   }
+  if (has) {
 #pragma unroll
-  for (int c = 0; c < R; c++) cell[c * LD] = {(T)s[c].x, (T)s[c].y};
+    for (int c = 0; c < R; c++) cell[c * LD] = {(T)s[c].x, (T)s[c].y};
+  }
   __syncthreads();
   if (t < S && !project) {
     double v = 0.0;
-    for (int w = 0; w < NT / 64; w++) v += wred[w][t];
+    for (int w = 0; w < NT / 16; w++) v += rowsum[w][t];
     partials[((long)inst * S + t) * a.nblk + blk] = v * a.inv_n;
   }
   fft_pencils<T, N, 1>(l, l, g, pen, 1 << 30, K::NPEN, fq, (T)-1, twl);
@@ -219,12 +423,16 @@ k_row_red(cx<T>* __restrict__ W, M xi, const RedArgs a, const RedOpt<T> o, const
 
 // ---------------------------------------------------------------- column kernel
 // Columns per block TC: row segments (R TC complex) of 128 to 192 bytes where
-// 48 KB of LDS allow it.
+// 48 KB of LDS allow it; about 256 k-points where N < 32.
 template <typename T, int N, int R> struct ColRed {
   static constexpr int TPP = make_plan(N).tpp, LD = pitch<N>();
   static constexpr size_t CSZ = sizeof(cx<T>);
   static constexpr int tc() {
     int t = 1;
+    if (N < 32) {
+      while (N * t * 2 <= 256 && t * 2 * R * TPP <= 512) t *= 2;
+      return t;
+    }
     while (t * 2 * R * CSZ <= 192 && (size_t)t * 2 * R * LD * CSZ <= 48 * 1024 && t * 2 * R * TPP <= 1024) t *= 2;
     return t;
   }
@@ -240,18 +448,6 @@ template <typename T, int N, int R> struct ColRed {
 // pass fold them to FOLD per field, and one block of the column kernel turns
 // those into the history row.  A field is added by one wave in a fixed order,
 // which is k_finish_sums' order for up to FOLD_ABOVE sums.
-constexpr int FOLD_ABOVE = 512;
-struct FoldJob {
-  const double* in;  // [F][nblk], null: nothing to fold
-  double* out;       // [F][FOLD]
-  int nblk, F;
-};
-struct FinishJob {
-  const double* in;  // [F][nblk], null: the sums are finished elsewhere
-  double* out;       // history
-  int* step_ctr;
-  int nblk, F, S;
-};
 __device__ __forceinline__ double wave_range_sum(const double* __restrict__ v, int b0, int b1) {
   double acc = 0.0;
   for (int b = b0 + ((int)threadIdx.x & 63); b < b1; b += 64) acc += v[b];
@@ -351,16 +547,17 @@ k_col_red(cx<T>* __restrict__ W, const ElasticConsts* __restrict__ ec, const T* 
     return;
   }
   const int t = threadIdx.x;
-  const long cols = P / N, tiles = cols / TC;
+  const long cols = P / N, tiles = (cols + TC - 1) / TC;
   const long bt = xcd_tile(blockIdx.x, blocks), inst = bt / tiles, m0 = (bt - inst * tiles) * TC;
   const int fp = t % NPEN, fq = t / NPEN;
-  const int pen = fq < TPP ? fp : 1 << 30;
+  const int nc = cols - m0 < TC ? (int)(cols - m0) : TC;  // columns of this block
+  const int pen = fq < TPP && fp < nc * R ? fp : 1 << 30;
   const StridedPencil<T> g{W + (inst * P + m0) * R + fp, cols * R};
   const LdsPencils<T> l{sm, LD};
   TwStage<T, N, NT> ts;
   ts.load(tw);
   fft_pencils<T, N, 1>(g, l, l, pen, 1 << 30, NPEN, fq, (T)-1, twl, [&] { ts.store(twl); });
-  for (int e = t; e < N * TC; e += NT) {
+  for (int e = t; e < N * nc; e += NT) {
     const int c = e / N, n = e % N;
     const long pt = (long)n * cols + m0 + c;
     if constexpr (STORED) contract_stored_lds<T, R>(sm + c * (R * LD) + n, LD, Kst + pt * (R * (R + 1) / 2));

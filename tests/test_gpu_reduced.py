@@ -130,3 +130,17 @@ def test_ensemble_class_equals_single(prec):
             x, ga = gpu(m, pa.PLAN_AUTO, prec, steps=19)
             assert np.array_equal(e.download_xi(i), x)
             assert np.abs(g[:, i] - ga.sum(1)).max() <= 1e-14
+
+
+SHORT = (2, 3, 4, 6, 8, 12, 16, 24)
+
+
+@pytest.mark.parametrize("prec", PRECS)
+@pytest.mark.parametrize("n", SHORT)
+def test_short_axes(n, prec):
+    """Lengths below 32 along N1 or N3, where blocks hold several rows or many
+    columns and N1 N2 rows (or N2 N3 columns) are no multiple of a block's."""
+    for shape, ns in (((n, 3, 32), 1), ((3, 6, n), 6), ((n, 2, 2), 12), ((48, 3, n), 3), ((2, 3, n), 4)):
+        w = C.small_fcc(shape, ns=ns, nloops=2, rmin=1.0, rmax=2.0)
+        bc, tau = options(w, ns == 6, ns == 4)
+        check(w, prec, bc=bc, tau=tau)
