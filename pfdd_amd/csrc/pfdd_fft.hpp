@@ -71,8 +71,24 @@ struct Plan {
 // with rlim = 4 the power of two is taken in radix-4 passes (and at most
 // one radix-2 pass): more passes, but twice the threads per pencil and half
 // the registers per thread.
+//
+// rlim = 16 (the reduced-basis kernels): two passes instead of three, with a
+// radix-6, 12 or 16 one, at 48, 96, 128, 192 and 256, and three instead of four
+// at 384; the other lengths as rlim = 8.  Each pass less is an LDS round trip
+// and a barrier less.  tpp covers the pass with the most butterflies.
 constexpr Plan make_plan(int n, int rlim = 8) {
   Plan p{};
+  if (rlim == 16) {
+    switch (n) {
+      case 48: return Plan{2, {8, 6}, 8};
+      case 96: return Plan{2, {8, 12}, 12};
+      case 128: return Plan{2, {8, 16}, 16};
+      case 192: return Plan{2, {12, 16}, 16};
+      case 256: return Plan{2, {16, 16}, 16};
+      case 384: return Plan{3, {8, 6, 8}, 64};
+      default: break;
+    }
+  }
   int m = n, rmax = 1;
   while (rlim >= 8 && m % 8 == 0) { p.r[p.np++] = 8; m /= 8; }
   if (rlim >= 8) {
@@ -157,6 +173,78 @@ template <typename T> struct Bfly<T, 8> {
     v[6] = csub<T>(e[2], o2);
     v[3] = cadd<T>(e[3], o3);
     v[7] = csub<T>(e[3], o3);
+  }
+};
+
+// The composite radices A x B: B transforms of A points, twiddles, A of B.
+// v[k1 + A k2] = sum_n2 w^(n2 k1) w_B^(n2 k2) sum_n1 v[B n1 + n2] w_A^(n1 k1)
+template <typename T> __device__ __forceinline__ cx<T> cmul_dir(cx<T> a, double c, double d, T s) {  // a (c + s i d)
+  const T x = (T)c, y = s * (T)d;
+  return {a.x * x - a.y * y, a.x * y + a.y * x};
+}
+template <typename T> struct Bfly<T, 6> {
+  __device__ __forceinline__ static void run(cx<T>* v, T s) {
+    cx<T> e[3] = {cadd<T>(v[0], v[3]), cadd<T>(v[1], v[4]), cadd<T>(v[2], v[5])};
+    cx<T> o[3] = {csub<T>(v[0], v[3]), csub<T>(v[1], v[4]), csub<T>(v[2], v[5])};
+    o[1] = cmul_dir<T>(o[1], 0.5, 0.86602540378443864676, s);   // w6
+    o[2] = cmul_dir<T>(o[2], -0.5, 0.86602540378443864676, s);  // w6^2
+    Bfly<T, 3>::run(e, s);
+    Bfly<T, 3>::run(o, s);
+#pragma unroll
+    for (int k = 0; k < 3; k++) v[2 * k] = e[k], v[2 * k + 1] = o[k];
+  }
+};
+template <typename T> struct Bfly<T, 12> {
+  __device__ __forceinline__ static void run(cx<T>* v, T s) {
+    constexpr double H = 0.86602540378443864676;
+    cx<T> a[3][4];
+#pragma unroll
+    for (int n = 0; n < 3; n++) {
+#pragma unroll
+      for (int m = 0; m < 4; m++) a[n][m] = v[3 * m + n];
+      Bfly<T, 4>::run(a[n], s);
+    }
+    a[1][1] = cmul_dir<T>(a[1][1], H, 0.5, s);   // w12
+    a[1][2] = cmul_dir<T>(a[1][2], 0.5, H, s);   // w12^2
+    a[1][3] = mul_si<T>(a[1][3], s);             // w12^3
+    a[2][1] = cmul_dir<T>(a[2][1], 0.5, H, s);   // w12^2
+    a[2][2] = cmul_dir<T>(a[2][2], -0.5, H, s);  // w12^4
+    a[2][3] = {-a[2][3].x, -a[2][3].y};          // w12^6
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      cx<T> b[3] = {a[0][k], a[1][k], a[2][k]};
+      Bfly<T, 3>::run(b, s);
+#pragma unroll
+      for (int m = 0; m < 3; m++) v[k + 4 * m] = b[m];
+    }
+  }
+};
+template <typename T> struct Bfly<T, 16> {
+  __device__ __forceinline__ static void run(cx<T>* v, T s) {
+    constexpr double C = 0.92387953251128675613, D = 0.38268343236508977173, Q = 0.70710678118654752440;
+    cx<T> a[4][4];
+#pragma unroll
+    for (int n = 0; n < 4; n++) {
+#pragma unroll
+      for (int m = 0; m < 4; m++) a[n][m] = v[4 * m + n];
+      Bfly<T, 4>::run(a[n], s);
+    }
+    a[1][1] = cmul_dir<T>(a[1][1], C, D, s);    // w16
+    a[1][2] = cmul_dir<T>(a[1][2], Q, Q, s);    // w16^2
+    a[1][3] = cmul_dir<T>(a[1][3], D, C, s);    // w16^3
+    a[2][1] = cmul_dir<T>(a[2][1], Q, Q, s);    // w16^2
+    a[2][2] = mul_si<T>(a[2][2], s);            // w16^4
+    a[2][3] = cmul_dir<T>(a[2][3], -Q, Q, s);   // w16^6
+    a[3][1] = cmul_dir<T>(a[3][1], D, C, s);    // w16^3
+    a[3][2] = cmul_dir<T>(a[3][2], -Q, Q, s);   // w16^6
+    a[3][3] = cmul_dir<T>(a[3][3], -C, -D, s);  // w16^9
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      cx<T> b[4] = {a[0][k], a[1][k], a[2][k], a[3][k]};
+      Bfly<T, 4>::run(b, s);
+#pragma unroll
+      for (int m = 0; m < 4; m++) v[k + 4 * m] = b[m];
+    }
   }
 };
 

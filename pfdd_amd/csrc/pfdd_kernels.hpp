@@ -684,10 +684,8 @@ __device__ __forceinline__ void contract_stress_form(const cx<T> (&v)[SM], const
 // registers.  No virtualevolv term (the GL steps).
 template <typename T, int S>
 __device__ __forceinline__ void contract_stress_form_lds(cx<T>* io, int stride, const ElasticConsts* __restrict__ ec,
-                                                         long pt) {
-  double f[3], g[6];
-  kvec(pt, ec, f);
-  if (!green6(f, ec, g)) {  // B(0) = 0
+                                                         const double f[3], const double g[6], bool nz) {
+  if (!nz) {  // B(0) = 0
 #pragma unroll
     for (int a = 0; a < S; a++) io[a * stride] = {(T)0, (T)0};
     return;
@@ -1425,7 +1423,10 @@ k_col_il_fixed(cx<T>* __restrict__ W, const ElasticConsts* __restrict__ ec, long
   fft((T)-1);
   for (int e = t; e < N * TC; e += NT) {
     const int c = e / N, n = e % N;  // consecutive threads read consecutive LDS words
-    contract_stress_form_lds<T, S>(sm + c * LD + lds_pos<SH>(n), TC * LD, ec, (long)n * M + m0 + c);
+    double f[3], g[6];
+    kvec((long)n * M + m0 + c, ec, f);
+    const bool nz = green6(f, ec, g);
+    contract_stress_form_lds<T, S>(sm + c * LD + lds_pos<SH>(n), TC * LD, ec, f, g, nz);
   }
   __syncthreads();
   fft((T)1);

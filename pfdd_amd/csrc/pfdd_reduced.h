@@ -8,6 +8,7 @@
 namespace pfdd {
 
 constexpr int RED_MAXR = 6;
+constexpr int RED_RL = 16;  // radix limit of these kernels' transforms
 
 // What the row kernel needs of the step (by value, read through the scalar cache).
 struct RedArgs {

@@ -69,10 +69,10 @@ template <typename T> bool col_any(const RedColLaunch<T>& q, int n1) {
 }
 #else
 template <typename T, int N> void pass2(const RedPass2Launch<T>& q) {
-  constexpr int TILE = tile_cols<T, N>(), NT = cols_threads<T, N>(), NW = NT / 64 > 0 ? NT / 64 : 1;
+  constexpr int TILE = tile_cols<T, N, RED_RL>(), NT = cols_threads<T, N, RED_RL>(), NW = NT / 64 > 0 ? NT / 64 : 1;
   const int blocks = (int)(q.outer * ((q.inner + TILE - 1) / TILE));
   const int nfold = q.fold.in ? (q.fold.F * FOLD + NW - 1) / NW : 0;
-  hipLaunchKernelGGL((k_pass2_red<T, N>), dim3((unsigned)(blocks + nfold)), dim3(NT), (cols_lds_bytes<T, N>()),
+  hipLaunchKernelGGL((k_pass2_red<T, N>), dim3((unsigned)(blocks + nfold)), dim3(NT), (cols_lds_bytes<T, N, RED_RL>()),
                      q.stream, q.W, (int)q.inner, blocks, (T)q.sign, q.tw, q.fold, nfold);
 }
 template <typename T> bool pass2_any(const RedPass2Launch<T>& q, int n2) {
@@ -86,9 +86,9 @@ template <typename T> bool pass2_any(const RedPass2Launch<T>& q, int n2) {
 }
 template <int N> bool pass2_attr() {
   return hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pass2_red<double, N>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)cols_lds_bytes<double, N>()) == hipSuccess &&
+                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)cols_lds_bytes<double, N, RED_RL>()) == hipSuccess &&
          hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pass2_red<float, N>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)cols_lds_bytes<float, N>()) == hipSuccess;
+                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)cols_lds_bytes<float, N, RED_RL>()) == hipSuccess;
 }
 #endif
 

@@ -66,7 +66,7 @@ __device__ __forceinline__ double row_sum4(const double (&v)[4]) {
 // and the transform may then need more lanes than there are points.  N1 N2 rows
 // need not be a multiple of ROWS: the last block may be short of rows.
 template <typename T, int N, int R, int PPT_> struct RowRed {
-  static constexpr int PPT = PPT_, ROWS = red_rows(N, PPT), PTS = ROWS * N, TPP = make_plan(N).tpp;
+  static constexpr int PPT = PPT_, ROWS = red_rows(N, PPT), PTS = ROWS * N, TPP = make_plan(N, RED_RL).tpp;
   static constexpr int LANES = ROWS * R * TPP, NEED = PTS / PPT > LANES ? PTS / PPT : LANES;
   static constexpr int NT = (NEED + 63) / 64 * 64;
   static constexpr int SH = 3, LD = padded_pitch<N, SH>(), NPEN = ROWS * R;
@@ -204,7 +204,7 @@ k_row_red(cx<T>* __restrict__ W, M xi, const RedArgs a, const RedOpt<T> o, const
   }
   const bool project = OPT && o.project;
   if (!project) {
-    fft_pencils<T, N, 1>(g, l, l, pen, 1 << 30, K::NPEN, fq, (T)1, twl, [&] { ts.store(twl); });
+    fft_pencils<T, N, 1, RED_RL>(g, l, l, pen, 1 << 30, K::NPEN, fq, (T)1, twl, [&] { ts.store(twl); });
   } else {
     ts.store(twl);
     __syncthreads();
@@ -282,7 +282,7 @@ k_row_red(cx<T>* __restrict__ W, M xi, const RedArgs a, const RedOpt<T> o, const
     for (int w = 0; w < NT / 16; w++) v += rowsum[w][t];
     partials[((long)inst * S + t) * a.nblk + blk] = v * a.inv_n;
   }
-  fft_pencils<T, N, 1>(l, l, g, pen, 1 << 30, K::NPEN, fq, (T)-1, twl);
+  fft_pencils<T, N, 1, RED_RL>(l, l, g, pen, 1 << 30, K::NPEN, fq, (T)-1, twl);
 }
 
 // plasticevolv (G.c:3485-3489) with the shear already divided by dslip.
@@ -344,7 +344,7 @@ k_row_red_n(cx<T>* __restrict__ W, M xi, const RedArgs a, const RedOpt<T> o, con
   }
   const bool project = OPT && o.project;
   if (!project) {
-    fft_pencils<T, N, 1>(g, l, l, pen, 1 << 30, K::NPEN, fq, (T)1, twl, [&] { ts.store(twl); });
+    fft_pencils<T, N, 1, RED_RL>(g, l, l, pen, 1 << 30, K::NPEN, fq, (T)1, twl, [&] { ts.store(twl); });
   } else {
     ts.store(twl);
     __syncthreads();
@@ -418,14 +418,18 @@ k_row_red_n(cx<T>* __restrict__ W, M xi, const RedArgs a, const RedOpt<T> o, con
     for (int w = 0; w < NT / 16; w++) v += rowsum[w][t];
     partials[((long)inst * S + t) * a.nblk + blk] = v * a.inv_n;
   }
-  fft_pencils<T, N, 1>(l, l, g, pen, 1 << 30, K::NPEN, fq, (T)-1, twl);
+  fft_pencils<T, N, 1, RED_RL>(l, l, g, pen, 1 << 30, K::NPEN, fq, (T)-1, twl);
 }
 
 // ---------------------------------------------------------------- column kernel
 // Columns per block TC: row segments (R TC complex) of 128 to 192 bytes where
 // 48 KB of LDS allow it; about 256 k-points where N < 32.
+// Radix limit: two passes (16) are faster in FP32 and, in FP64, at 48 and 96;
+// FP64's radix-16 pass at 128, 192 and 256 leaves half the lanes idle and
+// measured slower (128^3 x 3: 51 against 42 us, 256x256x192 x 3: 279 against 220).
 template <typename T, int N, int R> struct ColRed {
-  static constexpr int TPP = make_plan(N).tpp, LD = pitch<N>();
+  static constexpr int RL = sizeof(T) == 8 && N >= 128 ? 8 : RED_RL;
+  static constexpr int TPP = make_plan(N, RL).tpp, LD = pitch<N>();
   static constexpr size_t CSZ = sizeof(cx<T>);
   static constexpr int tc() {
     int t = 1;
@@ -439,6 +443,11 @@ template <typename T, int N, int R> struct ColRed {
   static constexpr int TC = tc(), NPEN = R * TC, LANES = (NPEN * TPP + 63) / 64 * 64;
   static constexpr int PTS = N * TC < 512 ? N * TC : 512;
   static constexpr int NT = LANES > PTS ? LANES : (PTS + 63) / 64 * 64;
+  static constexpr int KPT = (N * TC + NT - 1) / NT;  // k-points per thread
+  // The wave vectors are loaded with the tile in FP64 (256x256x192 x 3: 209
+  // against 223 us); in FP32 that measured slower (128^3 x 12: 45 against 42),
+  // and so it did in FP64 at 192 (192^3 x 3: 150 against 127).
+  static constexpr bool KEARLY = sizeof(T) == 8 && N % 3 != 0;
 };
 
 // The two stages of the per-field sums ride along as extra blocks of the
@@ -482,6 +491,33 @@ template <int NT> __device__ __forceinline__ void finish_block(const FinishJob& 
     j.step_ctr[0] = j.step_ctr[0] + 1;  // history row (read by every thread before the barrier above)
     j.step_ctr[1] = j.step_ctr[1] + 1;  // GL steps since the tau ramp was set
   }
+}
+
+// green6 with a reciprocal per distinct denominator (5 divisions instead of 25
+// for a cubic material; the same to rounding).
+__device__ __forceinline__ bool green6_rcp(const double f[3], const ElasticConsts* __restrict__ ec, double g[6]) {
+  const double a = f[0] * f[0], b = f[1] * f[1], c = f[2] * f[2], fk2 = a + b + c;
+  if (!(fk2 > 0.0)) return false;
+  const double inv = 1 / fk2;
+  double m0, m1, m2, w;  // 1 / m_i and (mu + lambda) / kk / |f|^2 of Bmatrix
+  if (ec->iso) {
+    m0 = m1 = m2 = ec->inv_mu;
+    w = ec->g_iso * ec->mu * ec->mu * inv;
+  } else {
+    const double mu = ec->mu, mup = ec->mup * inv, ml = ec->mu + ec->ll;
+    m0 = 1 / (mu + mup * a);
+    m1 = 1 / (mu + mup * b);
+    m2 = 1 / (mu + mup * c);
+    w = ml / (1.0 + ml * inv * (m0 * a + m1 * b + m2 * c)) * inv;
+  }
+  const double p0 = f[0] * m0, p1 = f[1] * m1, p2 = f[2] * m2;
+  g[0] = inv * (m0 - p0 * p0 * w);
+  g[1] = inv * (-p0 * p1 * w);
+  g[2] = inv * (-p0 * p2 * w);
+  g[3] = inv * (m1 - p1 * p1 * w);
+  g[4] = inv * (-p1 * p2 * w);
+  g[5] = inv * (m2 - p2 * p2 * w);
+  return true;
 }
 
 // Stored mode: K(k) as its upper triangle in the working precision, the
@@ -556,15 +592,31 @@ k_col_red(cx<T>* __restrict__ W, const ElasticConsts* __restrict__ ec, const T* 
   const LdsPencils<T> l{sm, LD};
   TwStage<T, N, NT> ts;
   ts.load(tw);
-  fft_pencils<T, N, 1>(g, l, l, pen, 1 << 30, NPEN, fq, (T)-1, twl, [&] { ts.store(twl); });
-  for (int e = t; e < N * nc; e += NT) {
-    const int c = e / N, n = e % N;
-    const long pt = (long)n * cols + m0 + c;
-    if constexpr (STORED) contract_stored_lds<T, R>(sm + c * (R * LD) + n, LD, Kst + pt * (R * (R + 1) / 2));
-    else contract_stress_form_lds<T, R>(sm + c * (R * LD) + n, LD, ec, pt);
+  double f[K::KPT][3];  // wave vectors of this thread's k-points
+  if constexpr (!STORED && K::KEARLY) {
+#pragma unroll
+    for (int k = 0; k < K::KPT; k++) {
+      const int e = t + k * NT, c = e / N;
+      kvec(c < nc ? (long)(e % N) * cols + m0 + c : 0, ec, f[k]);
+    }
+  }
+  fft_pencils<T, N, 1, K::RL>(g, l, l, pen, 1 << 30, NPEN, fq, (T)-1, twl, [&] { ts.store(twl); });
+#pragma unroll
+  for (int k = 0; k < K::KPT; k++) {
+    const int e = t + k * NT, c = e / N, n = e % N;
+    if (c >= nc) continue;
+    cx<T>* io = sm + c * (R * LD) + n;
+    if constexpr (STORED) {
+      contract_stored_lds<T, R>(io, LD, Kst + ((long)n * cols + m0 + c) * (R * (R + 1) / 2));
+    } else {
+      double gr[6];
+      if constexpr (!K::KEARLY) kvec((long)n * cols + m0 + c, ec, f[k]);
+      const bool nz = green6_rcp(f[k], ec, gr);
+      contract_stress_form_lds<T, R>(io, LD, ec, f[k], gr, nz);
+    }
   }
   __syncthreads();
-  fft_pencils<T, N, 1>(l, l, g, pen, 1 << 30, NPEN, fq, (T)1, twl);
+  fft_pencils<T, N, 1, K::RL>(l, l, g, pen, 1 << 30, NPEN, fq, (T)1, twl);
 }
 
 // ---------------------------------------------------------------- N2 pass
@@ -572,11 +624,11 @@ k_col_red(cx<T>* __restrict__ W, const ElasticConsts* __restrict__ ec, const T* 
 // k_fft_cols; the last tile of a row may be narrower than the others.
 // grid = fold blocks, then outer x tiles.
 template <typename T, int N>
-__global__ void __launch_bounds__((cols_threads<T, N>()))
+__global__ void __launch_bounds__((cols_threads<T, N, RED_RL>()))
 k_pass2_red(cx<T>* __restrict__ data, int inner, int blocks, T sign, const cx<T>* __restrict__ tw, const FoldJob fold,
             int nfold) {
-  constexpr int TILE = tile_cols<T, N>(), LD = pitch<N>(), NT = cols_threads<T, N>();
-  extern __shared__ unsigned char lds_raw[];  // cols_lds_bytes<T, N>()
+  constexpr int TILE = tile_cols<T, N, RED_RL>(), LD = pitch<N>(), NT = cols_threads<T, N, RED_RL>();
+  extern __shared__ unsigned char lds_raw[];  // cols_lds_bytes<T, N, RED_RL>()
   cx<T>* sm = reinterpret_cast<cx<T>*>(lds_raw);
   __shared__ cx<T> twl[N];
   if ((int)blockIdx.x < nfold) {
@@ -591,7 +643,7 @@ k_pass2_red(cx<T>* __restrict__ data, int inner, int blocks, T sign, const cx<T>
   const int i0 = (int)(bt - o * tiles) * TILE, np = inner - i0 < TILE ? inner - i0 : TILE;
   const ColPencils<T> g{data + o * N * inner + i0, inner};
   const LdsPencils<T> l{sm, LD};
-  fft_pencils<T, N, 1>(g, l, g, (int)threadIdx.x % TILE, 1 << 30, np, (int)threadIdx.x / TILE, sign, twl,
+  fft_pencils<T, N, 1, RED_RL>(g, l, g, (int)threadIdx.x % TILE, 1 << 30, np, (int)threadIdx.x / TILE, sign, twl,
                        [&] { ts.store(twl); });
 }
 
