@@ -14,7 +14,10 @@
 #include <cstdlib>
 #include <cstring>
 #include <algorithm>
+#include <atomic>
 #include <functional>
+#include <memory>
+#include <thread>
 #include <type_traits>
 #include <new>
 #include <vector>
@@ -44,6 +47,30 @@ struct Twiddles {
 
 }  // namespace
 
+// Pinned slots through which large device arrays reach the host: worker w
+// owns slot w and event w.  Allocated with the first large download, freed
+// with the last context that holds it.
+struct HostStage {
+  static constexpr int WORKERS = 6;
+  static constexpr size_t SLOT = 2 << 20;
+  char* base = nullptr;
+  hipEvent_t ev[WORKERS] = {};
+  int init() {
+    if (base) return PFDD_OK;
+    for (hipEvent_t& e : ev)
+      if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return PFDD_E_HIP;
+    void* p = nullptr;
+    if (hipHostMalloc(&p, SLOT * WORKERS, hipHostMallocDefault) != hipSuccess) return PFDD_E_ALLOC;
+    base = static_cast<char*>(p);
+    return PFDD_OK;
+  }
+  ~HostStage() {
+    if (base) (void)hipHostFree(base);
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
+  }
+};
+
 struct pfdd_ctx {
   pfdd_params p{};
   long P = 0;
@@ -67,7 +94,10 @@ struct pfdd_ctx {
   double2* taud = nullptr;   // [F] (tau, ramp rate)
   double* partials = nullptr;
   size_t partials_len = 0;
-  double* hist = nullptr;    // [HIST_CAP][B][S+1]
+  double* hist = nullptr;    // [HIST_CAP][B][S+1], in pinned host memory: the finish writes a row straight to the host
+  int hist_row = HIST_CAP;   // the host's copy of step_ctr[0]; HIST_CAP: not known, reset before use
+  int chunk_row = 0;         // history row of the running chunk's first step
+  std::shared_ptr<HostStage> stage;  // pinned slots of the large downloads, shared by the classes of an ensemble
   int* step_ctr = nullptr;
   double* small = nullptr;   // reduction outputs (<= 32 doubles)
   double* avepst_d = nullptr;
@@ -1166,8 +1196,13 @@ int strain_stress_impl(pfdd_ctx* c, const double* avepst_uniform, double* aveps,
   HIPCK(hipPeekAtLastError());
   double out[19];
   HIPCK(hipMemcpyAsync(out, c->small, sizeof(double) * 19, hipMemcpyDeviceToHost, c->stream));
-  if (eps_field) HIPCK(hipMemcpyAsync(eps_field, ef, sizeof(double) * 9 * P, hipMemcpyDeviceToHost, c->stream));
-  if (sig_field) HIPCK(hipMemcpyAsync(sig_field, sf, sizeof(double) * 9 * P, hipMemcpyDeviceToHost, c->stream));
+  for (int q = 0; q < 2; q++) {
+    double* dst = q ? sig_field : eps_field;
+    if (!dst) continue;
+    rc = read_points(c, (const char*)(q ? sf : ef), sizeof(double), nullptr, 0, 9 * (size_t)P,
+                     [&](size_t i, size_t m, const char* h, const char*) { memcpy(dst + i, h, sizeof(double) * m); });
+    if (rc) return rc;
+  }
   // restore the GL state: W must again hold the inverse-transformed data2
   // (the prologue has to be rerun by the caller if it had been done)
   HIPCK(hipStreamSynchronize(c->stream));
@@ -1201,11 +1236,12 @@ void pfdd_destroy(pfdd_ctx* c) {
   if (!c) return;
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   if (c->graph) (void)hipGraphExecDestroy(c->graph);
-  void* bufs[] = {c->xi,   c->W,        c->Bsym, c->mask, c->taupp, c->taud,   c->partials, c->hist,
+  void* bufs[] = {c->xi,   c->W,        c->Bsym, c->mask, c->taupp, c->taud,   c->partials,
                   c->step_ctr, c->small, c->avepst_d, c->ec, c->E6,  c->efield, c->sfield,   c->freq,
                   c->line_pts, c->line_out, c->Wr, c->Kst};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
+  if (c->hist) (void)hipHostFree(c->hist);
   for (auto& t : c->tw) {
     if (t.d) (void)hipFree(t.d);
     if (t.f) (void)hipFree(t.f);
@@ -1554,7 +1590,13 @@ int ctx_create(const pfdd_params* p, int batch, hipStream_t shared, pfdd_ctx** o
     if (!(c->xi = dev_alloc<char>(c->xi_bytes, c->bytes))) FAIL(PFDD_E_ALLOC);
     if (!(c->W = dev_alloc<char>(csz * F * P, c->bytes))) FAIL(PFDD_E_ALLOC);
     if (!(c->partials = (double*)dev_alloc<char>(sizeof(double) * c->partials_len, c->bytes))) FAIL(PFDD_E_ALLOC);
-    if (!(c->hist = (double*)dev_alloc<char>(sizeof(double) * HIST_CAP * c->B * (S + 1), c->bytes))) FAIL(PFDD_E_ALLOC);
+    if (hipHostMalloc((void**)&c->hist, sizeof(double) * HIST_CAP * c->B * (S + 1), hipHostMallocDefault) != hipSuccess)
+      FAIL(PFDD_E_ALLOC);
+    try {
+      c->stage = std::make_shared<HostStage>();
+    } catch (...) {
+      FAIL(PFDD_E_ALLOC);
+    }
     if (!(c->step_ctr = (int*)dev_alloc<char>(sizeof(int) * 4, c->bytes))) FAIL(PFDD_E_ALLOC);
     if (!(c->small = (double*)dev_alloc<char>(sizeof(double) * 32, c->bytes))) FAIL(PFDD_E_ALLOC);
     if (!(c->avepst_d = (double*)dev_alloc<char>(sizeof(double) * 9, c->bytes))) FAIL(PFDD_E_ALLOC);
@@ -1764,32 +1806,90 @@ int upload_inst(pfdd_ctx* c, int b, const double* xi, const double* xi_bc, int n
   return PFDD_OK;
 }
 
+// Reads n points from up to two device arrays (w0 and w1 bytes a point; d1 may
+// be null) and hands them to put(first point, points, array 0, array 1).
+// Large reads go through pinned slots and several threads, each of which
+// copies a stretch into its slot and then to its place: a single copy to
+// pageable memory, whose pages the reader has not touched yet, is bound by
+// one thread's page faults (128^3 x 12 FP64, 403 MB: 38 ms).
+constexpr size_t STAGE_ABOVE = 8 << 20;  // bytes; below, thread start-up costs what it saves
+template <typename Put>
+int read_points(pfdd_ctx* c, const char* d0, size_t w0, const char* d1, size_t w1, size_t n, Put&& put) {
+  HIPCK(hipStreamSynchronize(c->stream));
+  int dev = 0;
+  HIPCK(hipGetDevice(&dev));
+  const size_t w = w0 + w1;
+  if (n * w < STAGE_ABOVE || c->stage->init() != PFDD_OK) {
+    (void)hipGetLastError();
+    std::vector<char> h0(n * w0), h1(n * w1);
+    HIPCK(hipMemcpyAsync(h0.data(), d0, n * w0, hipMemcpyDeviceToHost, c->stream));
+    if (w1) HIPCK(hipMemcpyAsync(h1.data(), d1, n * w1, hipMemcpyDeviceToHost, c->stream));
+    HIPCK(hipStreamSynchronize(c->stream));
+    put(0, n, h0.data(), h1.data());
+    return PFDD_OK;
+  }
+  HostStage& st = *c->stage;
+  const size_t per = HostStage::SLOT / w / 16 * 16, nchunk = (n + per - 1) / per;
+  std::atomic<size_t> next{0};
+  std::atomic<int> rc{PFDD_OK};
+  auto work = [&](int id) {
+    if (hipSetDevice(dev) != hipSuccess) {
+      rc = PFDD_E_HIP;
+      return;
+    }
+    char* slot = st.base + (size_t)id * HostStage::SLOT;
+    for (size_t k; rc == PFDD_OK && (k = next++) < nchunk;) {
+      const size_t i = k * per, m = std::min(per, n - i);
+      if (hipMemcpyAsync(slot, d0 + i * w0, m * w0, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
+          (w1 && hipMemcpyAsync(slot + m * w0, d1 + i * w1, m * w1, hipMemcpyDeviceToHost, c->stream) != hipSuccess) ||
+          hipEventRecord(st.ev[id], c->stream) != hipSuccess || hipEventSynchronize(st.ev[id]) != hipSuccess) {
+        rc = PFDD_E_HIP;
+        return;
+      }
+      put(i, m, slot, slot + m * w0);
+    }
+  };
+  std::vector<std::thread> pool;
+  try {
+    pool.reserve(HostStage::WORKERS - 1);
+    for (int id = 1; id < HostStage::WORKERS; id++) pool.emplace_back(work, id);
+  } catch (...) {  // fewer threads: the ones there (or this one alone) do it all
+  }
+  work(0);
+  for (std::thread& t : pool) t.join();
+  return rc;
+}
+
 int download_inst(pfdd_ctx* c, int b, double* xi, int nsv) {
   if (!xi || nsv < c->S) return PFDD_E_SHAPE;
   const long P = c->P;
-  const size_t n = (size_t)c->S * P;
-  HIPCK(hipStreamSynchronize(c->stream));
+  const size_t n = (size_t)c->S * P, off = (size_t)b * n;
+  int rc;
   if (master64(c)) {
-    HIPCK(hipMemcpyAsync(xi, (double2*)c->xi + (size_t)b * n, sizeof(double2) * n, hipMemcpyDeviceToHost,
-                         c->stream));
-    HIPCK(hipStreamSynchronize(c->stream));
-  } else {
-    std::vector<float2> r(n);
-    const Master<float> m = xm<float>(c);
-    std::vector<float> im(m.im ? n : 0);
-    HIPCK(hipMemcpyAsync(r.data(), m.r + (size_t)b * n, sizeof(float2) * n, hipMemcpyDeviceToHost, c->stream));
-    if (m.im)
-      HIPCK(hipMemcpyAsync(im.data(), m.im + (size_t)b * n, sizeof(float) * n, hipMemcpyDeviceToHost, c->stream));
-    HIPCK(hipStreamSynchronize(c->stream));
-    for (size_t i = 0; i < n; i++) {
-      if (m.im) {
-        xi[2 * i] = (double)r[i].x + (double)r[i].y;
-        xi[2 * i + 1] = (double)im[i];
-      } else {
-        xi[2 * i] = (double)r[i].x;
-        xi[2 * i + 1] = (double)r[i].y;
-      }
+    const char* d = (const char*)c->xi + sizeof(double2) * off;
+    if (n * sizeof(double2) < STAGE_ABOVE) {
+      HIPCK(hipStreamSynchronize(c->stream));
+      HIPCK(hipMemcpyAsync(xi, d, sizeof(double2) * n, hipMemcpyDeviceToHost, c->stream));
+      HIPCK(hipStreamSynchronize(c->stream));
+    } else {
+      rc = read_points(c, d, sizeof(double2), nullptr, 0, n, [&](size_t i, size_t m, const char* h, const char*) {
+        memcpy(xi + 2 * i, h, sizeof(double2) * m);
+      });
+      if (rc) return rc;
     }
+  } else {
+    const Master<float> m = xm<float>(c);
+    rc = read_points(c, (const char*)(m.r + off), sizeof(float2), m.im ? (const char*)(m.im + off) : nullptr,
+                     m.im ? sizeof(float) : 0, n, [&](size_t i, size_t cnt, const char* h0, const char* h1) {
+                       const float2* r = (const float2*)h0;
+                       const float* im = (const float*)h1;
+                       double* x = xi + 2 * i;
+                       if (m.im)
+                         for (size_t k = 0; k < cnt; k++) x[2 * k] = (double)r[k].x + (double)r[k].y, x[2 * k + 1] = im[k];
+                       else
+                         for (size_t k = 0; k < cnt; k++) x[2 * k] = r[k].x, x[2 * k + 1] = r[k].y;
+                     });
+    if (rc) return rc;
   }
   if (nsv > c->S) memset(xi + 2 * n, 0, sizeof(double) * 2 * (size_t)(nsv - c->S) * P);
   return PFDD_OK;
@@ -1822,11 +1922,17 @@ int run_steps(pfdd_ctx* const* cs, int nc, hipStream_t st, hipGraphExec_t* graph
     return PFDD_OK;
   };
   int done = 0;
-  std::vector<double> h;
   while (done < nsteps) {
     const int chunk = std::min(HIST_CAP, nsteps - done);
-    for (int i = 0; i < nc; i++)
-      hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, st, cs[i]->step_ctr, 0);
+    for (int i = 0; i < nc; i++) {
+      // the history rows go on from the last call's; back to row 0 when the chunk would not fit
+      if (cs[i]->hist_row + chunk > HIST_CAP) {
+        hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, st, cs[i]->step_ctr, 0);
+        cs[i]->hist_row = 0;
+      }
+      cs[i]->chunk_row = cs[i]->hist_row;
+      cs[i]->hist_row = HIST_CAP;  // until the chunk is enqueued
+    }
     HIPCK(hipPeekAtLastError());
     int left = chunk;
     bool first = false;  // the first step after a prologue may take an argument that the others do not
@@ -1859,14 +1965,11 @@ int run_steps(pfdd_ctx* const* cs, int nc, hipStream_t st, hipGraphExec_t* graph
       const int rc = one();
       if (rc) return rc;
     }
+    for (int i = 0; i < nc; i++) cs[i]->hist_row = cs[i]->chunk_row + chunk;
     if (want_hist) {
-      for (int i = 0; i < nc; i++) {
-        const size_t row = (size_t)cs[i]->B * (cs[i]->S + 1);
-        h.resize((size_t)chunk * row);
-        HIPCK(hipMemcpyAsync(h.data(), cs[i]->hist, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st));
-        HIPCK(hipStreamSynchronize(st));
-        sink(i, done, chunk, h.data());
-      }
+      HIPCK(hipStreamSynchronize(st));
+      for (int i = 0; i < nc; i++)
+        sink(i, done, chunk, cs[i]->hist + (size_t)cs[i]->chunk_row * cs[i]->B * (cs[i]->S + 1));
     }
     done += chunk;
   }
@@ -1962,6 +2065,7 @@ int autotune_ctx(pfdd_ctx* c, int steps, int* best_plan, float* best_ms) {
   auto restore = [&]() -> int {
     HIPCK(hipMemcpyAsync(c->xi, xsave, xbytes, hipMemcpyDeviceToDevice, c->stream));
     HIPCK(hipMemcpyAsync(c->step_ctr, csave, sizeof(int) * 4, hipMemcpyDeviceToDevice, c->stream));
+    c->hist_row = HIST_CAP;
     HIPCK(hipStreamSynchronize(c->stream));
     return PFDD_OK;
   };
@@ -2152,7 +2256,7 @@ int pfdd_gl_steps_lines(pfdd_ctx* c, int nsteps, double* gamma, double* gamma_a,
     }
     rows.resize((size_t)n * F);
     if (copy_rc == PFDD_OK &&
-        (hipMemcpyAsync(rows.data(), c->line_out, sizeof(double) * rows.size(), hipMemcpyDeviceToHost, c->stream) !=
+        (hipMemcpyAsync(rows.data(), c->line_out + (size_t)c->chunk_row * F, sizeof(double) * rows.size(), hipMemcpyDeviceToHost, c->stream) !=
              hipSuccess ||
          hipStreamSynchronize(c->stream) != hipSuccess))
       copy_rc = PFDD_E_HIP;
@@ -2231,6 +2335,7 @@ int enqueue_stage(pfdd_ctx* c, int stage, int reps) {
         break;
       case PFDD_STAGE_STEP:
         hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, c->stream, c->step_ctr, 0);
+        c->hist_row = HIST_CAP;
         rc = c->ref32 ? ref32_step(c) : one_step<T>(c);
         break;
       case PFDD_STAGE_COPY:
@@ -2275,6 +2380,7 @@ extern "C" int pfdd_time_step_kernels(pfdd_ctx* c, int nsteps, float* ms, int* l
     if (hipEventCreateWithFlags(&e, hipEventDisableSystemFence) != hipSuccess) rc = PFDD_E_HIP;
   if (rc == PFDD_OK) {
     hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, c->stream, c->step_ctr, 0);
+    c->hist_row = HIST_CAP;
     taps.reserve(pool.size());
     c->tap_pool = &pool;
     c->tap = &taps;
@@ -2553,7 +2659,10 @@ int pfdd_create_ensemble(const pfdd_params* params, int count, pfdd_ens** out) {
     for (size_t k = 0; k < first.size() && rc == PFDD_OK; k++) {
       pfdd_ctx* c = nullptr;
       rc = ctx_create(&params[first[k]], size[k], e->stream, &c);
-      if (rc == PFDD_OK) e->cls.push_back(c);
+      if (rc == PFDD_OK) {
+        if (!e->cls.empty()) c->stage = e->cls[0]->stage;
+        e->cls.push_back(c);
+      }
     }
   }
   if (rc) {
@@ -2687,6 +2796,7 @@ int pfdd_ensemble_autotune(pfdd_ens* e, int steps, int* plans, float* ms_per_ste
       pfdd_ctx* c = e->cls[k];
       HIPCK(hipMemcpyAsync(c->xi, xsave[k], c->xi_bytes, hipMemcpyDeviceToDevice, e->stream));
       HIPCK(hipMemcpyAsync(c->step_ctr, csave[k], sizeof(int) * 4, hipMemcpyDeviceToDevice, e->stream));
+      c->hist_row = HIST_CAP;
     }
     HIPCK(hipStreamSynchronize(e->stream));
     return PFDD_OK;

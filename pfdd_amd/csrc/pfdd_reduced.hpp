@@ -473,19 +473,35 @@ template <int NT> __device__ __forceinline__ void fold_block(const FoldJob& j, i
   const double s = wave_range_sum(j.in + (long)f * j.nblk, b0, b0 + per < j.nblk ? b0 + per : j.nblk);
   if ((threadIdx.x & 63) == 0) j.out[(long)f * FOLD + part] = s;
 }
+// (The history row lies in host memory: it is written, never read back.)
+constexpr int FINISH_LDS = 64;  // fields whose sums the block holds in LDS
 template <int NT> __device__ __forceinline__ void finish_block(const FinishJob& j) {
   constexpr int NW = NT / 64;
-  const int ninst = j.F / j.S;
+  __shared__ double fsum[FINISH_LDS];
+  const int ninst = j.F / j.S, w = threadIdx.x >> 6;
   double* dst = j.out + (long)j.step_ctr[0] * ninst * (j.S + 1);
-  for (int f = threadIdx.x >> 6; f < j.F; f += NW) {
-    const double s = wave_range_sum(j.in + (long)f * j.nblk, 0, j.nblk);
-    if ((threadIdx.x & 63) == 0) dst[(f / j.S) * (j.S + 1) + f % j.S] = s;
-  }
-  __syncthreads();
-  for (int b = threadIdx.x; b < ninst; b += NT) {
-    double tot = 0.0;
-    for (int a = 0; a < j.S; a++) tot += dst[b * (j.S + 1) + a];
-    dst[b * (j.S + 1) + j.S] = tot;
+  if (j.F <= FINISH_LDS) {
+    for (int f = w; f < j.F; f += NW) {
+      const double s = wave_range_sum(j.in + (long)f * j.nblk, 0, j.nblk);
+      if ((threadIdx.x & 63) == 0) dst[(f / j.S) * (j.S + 1) + f % j.S] = fsum[f] = s;
+    }
+    __syncthreads();
+    for (int b = threadIdx.x; b < ninst; b += NT) {
+      double tot = 0.0;
+      for (int a = 0; a < j.S; a++) tot += fsum[b * j.S + a];
+      dst[b * (j.S + 1) + j.S] = tot;
+    }
+  } else {  // an instance per wave
+    for (int b = w; b < ninst; b += NW) {
+      double tot = 0.0;
+      for (int a = 0; a < j.S; a++) {
+        const double s = wave_range_sum(j.in + (long)(b * j.S + a) * j.nblk, 0, j.nblk);
+        if ((threadIdx.x & 63) == 0) dst[b * (j.S + 1) + a] = s;
+        tot += s;
+      }
+      if ((threadIdx.x & 63) == 0) dst[b * (j.S + 1) + j.S] = tot;
+    }
+    __syncthreads();
   }
   if (threadIdx.x == 0) {
     j.step_ctr[0] = j.step_ctr[0] + 1;  // history row (read by every thread before the barrier above)
