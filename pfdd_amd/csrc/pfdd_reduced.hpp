@@ -198,6 +198,23 @@ k_row_red(cx<T>* __restrict__ W, M xi, const RedArgs a, const RedOpt<T> o, const
       for (int p = 0; p < PPT; p++)  // (a lane without a point loads the block's first)
         raw[p][f] = m.raw(t + p * NT < nr * N ? t + p * NT : 0);
     }
+  // the options' arrays, loaded with the master: the per-point shear (over
+  // dslip) or the uniform one, and the frozen flags as bits
+  double pq[OPT ? PPT : 1][OPT ? SM : 1];
+  unsigned frozen[OPT ? PPT : 1];
+  if constexpr (OPT) {
+#pragma unroll
+    for (int p = 0; p < PPT; p++) {
+      const int e0 = t + p * NT < nr * N ? t + p * NT : 0;
+      frozen[p] = 0;
+#pragma unroll
+      for (int f = 0; f < SM; f++) {
+        if (f >= S) continue;
+        if (o.taupp) pq[p][f] = o.taupp[((long)inst * P + pt0 + e0) * S + f];
+        if (o.mask) frozen[p] |= (o.mask[x0 + (long)f * P + e0] ? 1u : 0u) << f;
+      }
+    }
+  }
   if (t < S) {
     const double2 tr = a.tau[inst * S + t];
     tq[t] = (tr.x + tr.y * (double)step_ctr[1]) / a.dslip[t];
@@ -245,10 +262,8 @@ k_row_red(cx<T>* __restrict__ W, M xi, const RedArgs a, const RedOpt<T> o, const
             dr += (double)v.x;
             di += (double)v.y;
           }
-          if (o.taupp)
-            q = (o.taupp[((long)inst * P + pt0 + e0) * S + f] + a.tau[inst * S + f].y * (double)step_ctr[1]) /
-                a.dslip[f];
-          if (o.mask) live = o.mask[e] == 0;
+          if (o.taupp) q = (pq[p][f] + a.tau[inst * S + f].y * (double)step_ctr[1]) / a.dslip[f];
+          live = !((frozen[p] >> f) & 1);
         }
         if (live) {
           const double arg = a.two_pi * x.x;
@@ -473,17 +488,39 @@ template <int NT> __device__ __forceinline__ void fold_block(const FoldJob& j, i
   const double s = wave_range_sum(j.in + (long)f * j.nblk, b0, b0 + per < j.nblk ? b0 + per : j.nblk);
   if ((threadIdx.x & 63) == 0) j.out[(long)f * FOLD + part] = s;
 }
+// The sums of fields f0 .. f0 + 3 (clamped to the last), their loads and
+// exchanges in flight together: one field at a time, the 12 fields of a
+// 32^3 grid took one wave 12 us, longer than the rest of the column kernel.
+__device__ __forceinline__ void wave_sums4(const FinishJob& j, int f0, double (&s)[4]) {
+  const double* v[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    v[i] = j.in + (long)(f0 + i < j.F ? f0 + i : j.F - 1) * j.nblk;
+    s[i] = 0.0;
+  }
+  for (int b = (int)threadIdx.x & 63; b < j.nblk; b += 64)
+#pragma unroll
+    for (int i = 0; i < 4; i++) s[i] += v[i][b];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+    for (int i = 0; i < 4; i++) s[i] += __shfl_xor(s[i], o, 64);
+}
 // (The history row lies in host memory: it is written, never read back.)
 constexpr int FINISH_LDS = 64;  // fields whose sums the block holds in LDS
 template <int NT> __device__ __forceinline__ void finish_block(const FinishJob& j) {
   constexpr int NW = NT / 64;
   __shared__ double fsum[FINISH_LDS];
   const int ninst = j.F / j.S, w = threadIdx.x >> 6;
+  const bool lane0 = (threadIdx.x & 63) == 0;
   double* dst = j.out + (long)j.step_ctr[0] * ninst * (j.S + 1);
+  double s[4];
   if (j.F <= FINISH_LDS) {
-    for (int f = w; f < j.F; f += NW) {
-      const double s = wave_range_sum(j.in + (long)f * j.nblk, 0, j.nblk);
-      if ((threadIdx.x & 63) == 0) dst[(f / j.S) * (j.S + 1) + f % j.S] = fsum[f] = s;
+    for (int f0 = 4 * w; f0 < j.F; f0 += 4 * NW) {
+      wave_sums4(j, f0, s);
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (lane0 && f0 + i < j.F) dst[(f0 + i) / j.S * (j.S + 1) + (f0 + i) % j.S] = fsum[f0 + i] = s[i];
     }
     __syncthreads();
     for (int b = threadIdx.x; b < ninst; b += NT) {
@@ -494,12 +531,16 @@ template <int NT> __device__ __forceinline__ void finish_block(const FinishJob& 
   } else {  // an instance per wave
     for (int b = w; b < ninst; b += NW) {
       double tot = 0.0;
-      for (int a = 0; a < j.S; a++) {
-        const double s = wave_range_sum(j.in + (long)(b * j.S + a) * j.nblk, 0, j.nblk);
-        if ((threadIdx.x & 63) == 0) dst[b * (j.S + 1) + a] = s;
-        tot += s;
+      for (int a0 = 0; a0 < j.S; a0 += 4) {
+        wave_sums4(j, b * j.S + a0, s);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          if (a0 + i >= j.S) continue;
+          if (lane0) dst[b * (j.S + 1) + a0 + i] = s[i];
+          tot += s[i];
+        }
       }
-      if ((threadIdx.x & 63) == 0) dst[b * (j.S + 1) + j.S] = tot;
+      if (lane0) dst[b * (j.S + 1) + j.S] = tot;
     }
     __syncthreads();
   }
