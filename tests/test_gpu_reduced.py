@@ -144,3 +144,32 @@ def test_short_axes(n, prec):
         w = C.small_fcc(shape, ns=ns, nloops=2, rmin=1.0, rmax=2.0)
         bc, tau = options(w, ns == 6, ns == 4)
         check(w, prec, bc=bc, tau=tau)
+
+
+@pytest.mark.parametrize("sizes", [(16, 32), (16, 24, 32, 48, 12, 8)])
+def test_classes_on_parallel_branches(sizes):
+    """Fewer and more classes than a graph has branches, in different
+    precisions; replays, eager steps between them and a new prologue:
+    bit-identical to each instance alone."""
+    ws = [C.small_fcc((n, n, n), ns=1 + k % 4, seed=C.BASE_SEED + 700 + k) for k, n in enumerate(sizes)]
+    precs = [PRECS[k % 3] for k in range(len(ws))]
+    calls = (19, 8, 3, 17)
+    with pa.Ensemble([w.params(p) for w, p in zip(ws, precs)]) as e:
+        for i, w in enumerate(ws):
+            e.set_tau(i, w.tau)
+            e.upload_xi(i, w.xi)
+        g = []
+        for n in calls:
+            e.begin_outer(True)
+            g.append(e.gl_steps(n))
+        got = [e.download_xi(i) for i in range(len(ws))]
+    for i, (w, p) in enumerate(zip(ws, precs)):
+        with pa.Context(w.params(p)) as c:
+            c.set_tau(w.tau)
+            c.upload_xi(w.xi)
+            gs = []
+            for n in calls:
+                c.begin_outer(True)
+                gs.append(c.gl_steps(n)[0])
+            assert np.array_equal(c.download_xi(), got[i]), i
+        assert np.array_equal(np.concatenate(gs), np.concatenate(g)[:, i]), i
