@@ -78,8 +78,12 @@ typedef struct {
 } pfdd_params;
 
 /* Kernel plan word (no reference counterpart; results are the same to
- * rounding for every plan).  AUTO picks the plan measured fastest at
- * 128^3 x 12; pfdd_autotune measures the candidates on the actual problem.
+ * rounding for every plan).  AUTO steps in a basis of the eigenstrains: the
+ * transforms and the contraction run on its R <= min(ns, 6) components, which
+ * the update kernel forms from the ns fields.  Any other word runs on the slip
+ * fields themselves, AUTO too when there is no memory for the components;
+ * with PFDD_B_STORED each builds its own form of B(k) on first use.
+ * pfdd_autotune measures the candidates on the actual problem.
  * Bits 0-4 are flags; bits 8-11 and 12-15 optionally fix the tile of the
  * fused row / column kernel as log2(tile) + 1 (0 = the largest that fits);
  * a tile that does not fit is rejected with PFDD_E_SHAPE; bits 16-18 pick
@@ -89,7 +93,7 @@ enum {
   PFDD_PLAN_UNFUSED_ROWS = 1,  /* plain N3 passes + pointwise update instead of the fused row kernel */
   PFDD_PLAN_UNFUSED_COLS = 2,  /* plain N1 passes + pointwise contraction instead of the fused column kernel */
   PFDD_PLAN_FUSED_COLS = 4,    /* fused column kernel whenever its tile fits in LDS */
-  PFDD_PLAN_NO_PLANE = 8,      /* no LDS-resident N2 x N3 plane kernel (AUTO uses it for N2 = N3 <= 96) */
+  PFDD_PLAN_NO_PLANE = 8,      /* no LDS-resident N2 x N3 plane kernel (plans on slip fields use it for N2 = N3 <= 96) */
   PFDD_PLAN_PLANE = 16,        /* the plane kernel also at 128^2 (mixed precision only) */
   PFDD_PLAN_ROW_TILE_SHIFT = 8,  /* rows along N3 per block of the fused row kernel */
   PFDD_PLAN_COL_TILE_SHIFT = 12, /* (i2,i3) columns per block of the fused column kernel */
@@ -282,7 +286,8 @@ int pfdd_ensemble_set_plan(pfdd_ens *e, int cls, int plan);
  * hipGraph.  Persistent mode needs every class cubic with N in
  * {32,48,64,96}, ns <= 4, recomputed B, no frozen points and uniform shear
  * (PFDD_E_UNSUPPORTED otherwise); it sets each class's plan to
- * PFDD_PLAN_PLANE | PFDD_PLAN_FUSED_COLS.  Both modes give the same bits.
+ * PFDD_PLAN_PLANE | PFDD_PLAN_FUSED_COLS and gives the bits of the phased
+ * mode with that plan.
  * A completion wait is bounded (about 2 s); one that runs out skips its item
  * and makes the next synchronous call (pfdd_ensemble_gl_steps with gamma,
  * pfdd_ensemble_sync) return PFDD_E_HIP.

@@ -1338,13 +1338,18 @@ int build_stored(pfdd_ctx* c) {
   return hipPeekAtLastError() == hipSuccess ? PFDD_OK : PFDD_E_HIP;
 }
 
-// Whether AUTO runs the steps in the reduced basis.
+// Whether AUTO runs the steps in the reduced basis: everywhere, since it moves
+// 8 R + 2 S complex values a point and step where the plans on slip fields move
+// 8 S + 2 S, R <= min(S, 6) (128^3 x 12 FP64: 342 against 679 us a step, 32^3 x 3:
+// 17.4 against 33), but for one range: on slabs of N2 <= 8 whose lengths have
+// compile-time interleaved kernels, AUTO's results are promised to be those of
+// the field-major plan to the last bit.  It is not the faster side there: us a
+// step, interleaved or field-major against reduced, (128,8,128) x 12 FP64 66
+// against 54, (256,8,256) x 12 FP64 244 against 113 and lean 119 against 76.
 bool auto_reduced(const pfdd_ctx* c, int plan) {
   const pfdd_params& p = c->p;
   if (plan != PFDD_PLAN_AUTO) return false;
-  const size_t csz = c->fp64 ? sizeof(double2) : sizeof(float2);
-  if (!c->stored && p.n1 == p.n3 && il_fixed_S(p.n1) == c->S && csz * c->S * c->P <= (128u << 20)) return false;
-  return true;
+  return c->stored || p.n2 > 8 || p.n1 != p.n3 || il_fixed_S(p.n1) != c->S;
 }
 
 // The work array of the reduced basis (and K(k) in stored mode), on first
@@ -1424,7 +1429,7 @@ int apply_plan(pfdd_ctx* c, int plan) {
     const int rc = build_stored(c);
     if (rc) return rc;
   }
-  // AUTO takes the interleaved layout where its compile-time row and column
+  // On the slip fields AUTO takes the interleaved layout where its compile-time row and column
   // kernels exist (S = 12 at N1 = N3 = 128 or 256, S = 3 at 512; recomputed
   // B) and measured faster than the field-major plan: at 128^3 x 12 0.686
   // against 0.909 ms per FP64 step and 0.400 against 0.466 ms per mixed
