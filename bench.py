@@ -25,63 +25,49 @@ from pfdd_amd import hip  # noqa: E402
 
 METRIC = "GL steps/s at 128^3×12 slip, FP64 vs mixed FP32 at stated error; % HBM peak"
 HBM_PEAK_GBS = 8000.0
-STAGES = [("k_update", pa.STAGE_UPDATE, 1), ("k_fft_rows(N3)", pa.STAGE_FFT_AXIS3, 2),
-          ("k_fft_cols(N2)", pa.STAGE_FFT_AXIS2, 2), ("k_fft_cols(N1)", pa.STAGE_FFT_AXIS1, 2),
-          ("k_contract", pa.STAGE_CONTRACT, 1)]
+# The AUTO plan: the R component fields of a basis of the eigenstrains (5 for
+# the 12 FCC systems) are transformed in place of the S slip fields.
+STAGES = [("k_row_red(N3 inv + update + N3 fwd)", pa.STAGE_UPDATE), ("k_pass2_red(N2)", pa.STAGE_FFT_AXIS2),
+          ("k_col_red(N1 fwd + B(k) + N1 inv)", pa.STAGE_CONTRACT), ("k_finish_sums", pa.STAGE_FINISH)]
 
 
-def stage_bytes(stage, S, P, ntri, fp64, stored, lean=False):
+def basis_size(w):
+    """Dimensions the symmetric eigenstrains span: the components transformed."""
+    e = np.asarray(w.eps, dtype=np.float64).reshape(w.ns, 3, 3)
+    return int(np.linalg.matrix_rank((0.5 * (e + e.transpose(0, 2, 1))).reshape(w.ns, 9)))
+
+
+def master_bytes(fp64, lean):
+    return 16 if fp64 else 8 if lean else 12      # double2, plain FP32 or the compensated FP32 form
+
+
+def stage_bytes(stage, S, R, P, fp64, stored, lean=False):
     """Algorithmic bytes of one launch: each input read once, each output written once."""
-    c = 16 if fp64 else 8
-    m = 16 if fp64 else 8 if lean else 12         # master xi: double2, plain FP32 or the compensated FP32 form
+    c, m = 16 if fp64 else 8, master_bytes(fp64, lean)
     if stage == pa.STAGE_FINISH:
         return 0
-    r = 8 if fp64 else 4
     if stage == pa.STAGE_UPDATE:
-        return S * P * (c + m + m + c)            # read W, read xi, write xi, write W
-    if stage in (pa.STAGE_FFT_AXIS3, pa.STAGE_FFT_AXIS2, pa.STAGE_FFT_AXIS1):
-        return S * P * 2 * c
+        return P * (2 * R * c + 2 * S * m)        # read W, read xi, write xi, write W
+    if stage == pa.STAGE_FFT_AXIS2:
+        return P * 2 * R * c
     if stage == pa.STAGE_CONTRACT:
-        return S * P * 2 * c + (ntri * P * r if stored else 0)
+        return P * (2 * R * c + (R * (R + 1) // 2 * (c // 2) if stored else 0))
     if stage == pa.STAGE_COPY:
         return S * P * (m + c)
     raise ValueError(stage)
 
 
-def fixed_interleaved(shape, S, stored):
-    """AUTO runs the interleaved layout with the compile-time row and column
-    kernels (k_row_il_fixed, k_col_il_fixed) for S = 12 at N1 = N3 = 128 with
-    recomputed B (apply_plan in pfdd_api.hip)."""
-    return S == 12 and shape[0] == 128 and shape[2] == 128 and not stored
-
-
-def rocprof_name(stage, plan, fp64, shape, S, stored, lean=False):
+def rocprof_name(stage, fp64, shape, S, R, stored, lean=False):
     """The kernel symbol rocprofv3 reports for a stage of this context (AUTO plan)."""
     T = "double" if fp64 else "float"
-    M = "pfdd::Master<double> " if fp64 else "pfdd::MasterF32L" if lean else "pfdd::MasterF32C"
+    M = "pfdd::Master<double>" if fp64 else "pfdd::MasterF32L" if lean else "pfdd::MasterF32C"
     n1, n2, n3 = shape
-    sm = 4 if S <= 4 else 8 if S <= 8 else 12 if S <= 12 else 16
-    if fixed_interleaved(shape, S, stored):
-        if stage == pa.STAGE_UPDATE:
-            return f"void pfdd::k_row_il_fixed<{T}, {n3}, 12, 1, {M}>"
-        if stage == pa.STAGE_CONTRACT:
-            return f"void pfdd::k_col_il_fixed<{T}, {n1}, 12, {1 if fp64 else 2}>"
-        if stage == pa.STAGE_FFT_AXIS2:
-            return f"void pfdd::k_fft_cols<{T}, {n2}, 8, false>"
-        return None
-    if stage == pa.STAGE_UPDATE:
-        return (f"void pfdd::k_row_step<{T}, {n3}, false, false, {M}>" if plan[pa.STAGE_FFT_AXIS3] == 0
-                else f"void pfdd::k_update<{T}, false, false>")
-    # (the AUTO plan: radix-8 sequences, field-major layout, narrow column tiles)
-    if stage == pa.STAGE_FFT_AXIS3:
-        return f"void pfdd::k_fft_rows<{T}, {n3}, 8>"
+    if stage == pa.STAGE_UPDATE and R > 4:
+        return f"void pfdd::k_row_red_n<{T}, {n3}, {R}, {M}, false>"
     if stage == pa.STAGE_FFT_AXIS2:
-        return f"void pfdd::k_fft_cols<{T}, {n2}, 8, false>"
-    if stage == pa.STAGE_FFT_AXIS1:
-        return f"void pfdd::k_fft_cols<{T}, {n1}, 8, false>"
+        return f"void pfdd::k_pass2_red<{T}, {n2}>"
     if stage == pa.STAGE_CONTRACT:
-        return (f"void pfdd::k_col_contract<{T}, {n1}, {sm}>" if plan[pa.STAGE_FFT_AXIS1] == 0
-                else f"void pfdd::k_contract<{T}, {sm}, {'true' if stored else 'false'}, false>")
+        return f"void pfdd::k_col_red<{T}, {n1}, {R}, {'true' if stored else 'false'}>"
     return None
 
 
@@ -98,13 +84,12 @@ def measured_traffic(name):
     return None if k is None else int(round(k["traffic_bytes"]))
 
 
-def step_alg_bytes(S, P, fp64, stored, lean=False):
-    """Stage-minimum bytes of one GL step (C2C, FP64: (144 S [+4 S(S+1)]) P;
-    mixed with the 12-byte compensated master: (88 S [+2 S(S+1)]) P; with the
-    8-byte plain FP32 master: (80 S [+2 S(S+1)]) P)."""
-    if fp64:
-        return (144 * S + (4 * S * (S + 1) if stored else 0)) * P
-    return ((80 if lean else 88) * S + (2 * S * (S + 1) if stored else 0)) * P
+def step_alg_bytes(S, R, P, fp64, stored, lean=False):
+    """Bytes of one GL step, each kernel's inputs read once and outputs written
+    once (FP64: (128 R + 32 S) P, mixed (64 R + 24 S) P, lean (64 R + 16 S) P)."""
+    return (stage_bytes(pa.STAGE_UPDATE, S, R, P, fp64, stored, lean)
+            + 2 * stage_bytes(pa.STAGE_FFT_AXIS2, S, R, P, fp64, stored)
+            + stage_bytes(pa.STAGE_CONTRACT, S, R, P, fp64, stored))
 
 
 # GL steps per captured hipGraph chunk (GRAPH_STEPS in pfdd_api.hip): the
@@ -142,14 +127,7 @@ def time_kernels(ctx, nsteps=20):
     from HIP events recorded between the launches of nsteps eager GL steps on
     the context's stream (pfdd_time_step_kernels), so every launch is timed in
     the sequence it runs in during a step."""
-    plan = ctx.step_plan()
-    names = {st: n for n, st, _ in STAGES}
-    names[pa.STAGE_FINISH] = "k_finish_sums"
-    fixed = fixed_interleaved(ctx.shape, ctx.ns, ctx.params.bmode == pa.B_STORED)
-    if plan[pa.STAGE_FFT_AXIS3] == 0:
-        names[pa.STAGE_UPDATE] = ("k_row_il_fixed" if fixed else "k_row_step") + "(N3 inv + update + N3 fwd)"
-    if plan[pa.STAGE_FFT_AXIS1] == 0:
-        names[pa.STAGE_CONTRACT] = ("k_col_il_fixed" if fixed else "k_col_contract") + "(N1 fwd + B(k) + N1 inv)"
+    names = {st: n for n, st in STAGES}
     out = {}
     for st, (ms, n) in ctx.time_step_kernels(nsteps).items():
         out[names[st]] = (st, n, ms / n)
@@ -246,8 +224,7 @@ def main():
     bmode = pa.B_RECOMPUTE if a.bmode == "recompute" else pa.B_STORED
     stored = bmode == pa.B_STORED
     w = C.c1(bmode)
-    S, P = w.ns, w.P
-    ntri = S * (S + 1) // 2
+    S, R, P = w.ns, basis_size(w), w.P
 
     # ---- FP64 (value)
     progress("FP64 timed steps")
@@ -255,7 +232,6 @@ def main():
     ms64, wall64, wu = timed_steps(ctx, a.steps, a.warmup)
     stages = time_kernels(ctx)
     copy_ms = copy_reference(ctx)
-    plan = ctx.step_plan()
     ctx.close()
     sps64 = a.steps / (ms64 / 1e3)
 
@@ -263,19 +239,19 @@ def main():
     dom = max(((n, st, k, ms) for n, (st, k, ms) in stages.items() if k > 0 and st != pa.STAGE_FINISH),
               key=lambda t: t[2] * t[3])
     dname, dst, _, dms = dom
-    dbytes = stage_bytes(dst, S, P, ntri, True, stored)
+    dbytes = stage_bytes(dst, S, R, P, True, stored)
     achieved = dbytes / (dms / 1e3) / 1e9
-    rname = rocprof_name(dst, plan, True, w.shape, S, stored)
+    rname = rocprof_name(dst, True, w.shape, S, R, stored)
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": measured_traffic(rname), "kernel": dname,
                 "rocprof_kernel": rname, "alg_bytes_per_launch": dbytes, "avg_launch_ms": round(dms, 5)}
-    step_bytes = step_alg_bytes(S, P, True, stored)
+    step_bytes = step_alg_bytes(S, R, P, True, stored)
     step_gbs = step_bytes * sps64 / 1e9
     kernels = {n: {"avg_ms": round(ms, 5), "launches_per_step": k,
-                   "GB_s": round(stage_bytes(st, S, P, ntri, True, stored) / (ms / 1e3) / 1e9, 1)}
+                   "GB_s": round(stage_bytes(st, S, R, P, True, stored) / (ms / 1e3) / 1e9, 1)}
                for n, (st, k, ms) in stages.items()}
     kernels["k_xi_to_w(copy reference)"] = {"avg_ms": round(copy_ms, 5), "launches_per_step": 0,
-                                            "GB_s": round(stage_bytes(pa.STAGE_COPY, S, P, ntri, True, stored)
+                                            "GB_s": round(stage_bytes(pa.STAGE_COPY, S, R, P, True, stored)
                                                           / (copy_ms / 1e3) / 1e9, 1)}
 
     out = {"metric": METRIC, "value": round(sps64, 2), "unit": "GL steps/s", "n_gpus": 1, "steps": a.steps,
@@ -284,7 +260,7 @@ def main():
            "data": "synthetic: seeded loops (SplitMix64, seed 20261202+1), sigma_ij ~ U[-0.02,0.02]",
            "config": {"workload": "c1: 128^3 grid x 12 FCC slip systems, 16 seeded circular loops r~U[5,20], "
                                   "FP64 GL step (FFT + B(k) contraction + update)",
-                      "grid": [128, 128, 128], "ns": S, "precision": "fp64", "bmode": a.bmode,
+                      "grid": [128, 128, 128], "ns": S, "basis_components": R, "precision": "fp64", "bmode": a.bmode,
                       "parallelism": "single GPU"},
            "roofline": roofline,
            "step_roofline": {"alg_bytes_per_step": step_bytes, "achieved_GB_s": round(step_gbs, 1),
@@ -304,10 +280,10 @@ def main():
         out[key] = {"value": round(sps32, 2), "unit": "GL steps/s", "speedup_vs_fp64": round(sps32 / sps64, 3),
                     "ms_per_step": round(ms32 / a.steps, 5),
                     "master_xi": "plain FP32 complex, 8 B" if lean else "compensated FP32 (hi + lo, im), 12 B",
-                    "step_roofline_frac": round(step_alg_bytes(S, P, False, stored, lean) * sps32 / 1e9
+                    "step_roofline_frac": round(step_alg_bytes(S, R, P, False, stored, lean) * sps32 / 1e9
                                                 / HBM_PEAK_GBS, 4),
                     "kernels": {n: {"avg_ms": round(ms, 5), "launches_per_step": k,
-                                    "GB_s": round(stage_bytes(st, S, P, ntri, False, stored, lean)
+                                    "GB_s": round(stage_bytes(st, S, R, P, False, stored, lean)
                                                   / (ms / 1e3) / 1e9, 1)}
                                 for n, (st, k, ms) in stages32.items()}}
 

@@ -155,12 +155,14 @@ def run_ensemble(w, steps, precision, tune_steps=8):
     return out, e
 
 
-def step_bytes(S, P, fp64, stored, lean=False):
-    """Stage-minimum bytes of a GL step (the mixed master xi takes 12 bytes a
-    point, 8 in the lean form)."""
-    if fp64:
-        return (144 * S + (4 * S * (S + 1) if stored else 0)) * P
-    return ((80 if lean else 88) * S + (2 * S * (S + 1) if stored else 0)) * P
+def step_bytes(eps, P, fp64, stored, lean=False):
+    """Bytes of a GL step, each kernel's inputs read once and outputs written
+    once: eight passes over the R basis components and one read and one write
+    of the master xi (12 bytes a point in the mixed mode, 8 in the lean form)."""
+    e = np.asarray(eps, dtype=np.float64).reshape(-1, 3, 3)
+    S, R = len(e), int(np.linalg.matrix_rank((0.5 * (e + e.transpose(0, 2, 1))).reshape(-1, 9)))
+    m, c = (16, 16) if fp64 else (8 if lean else 12, 8)
+    return (8 * R * c + 2 * S * m + (R * (R + 1) // 2 * (c // 2) if stored else 0)) * P
 
 
 def main():
@@ -188,7 +190,7 @@ def main():
                                         slipped_area_rel_err=float(abs(gar[-1].sum() * w.P - ga64[-1].sum() * w.P)
                                                                    / abs(ga64[-1].sum() * w.P)),
                                         mean_stress_max_abs_err=float(np.abs(sr - s64).max()),
-                                        step_roofline_frac=step_bytes(w.ns, w.P, False, False) * rr["steps_per_s"] / 8e12)
+                                        step_roofline_frac=step_bytes(w.eps, w.P, False, False) * rr["steps_per_s"] / 8e12)
         del xr
         rl, xl, gal, el, sl = run_plain(w, steps, MIXED_LEAN, B_RECOMPUTE)
         print(f"[run_config] mixed lean (FP32 master) recomputed B {rl['steps_per_s']:.2f} steps/s", flush=True)
@@ -197,7 +199,7 @@ def main():
                                              slipped_area_rel_err=float(abs(gal[-1].sum() - ga64[-1].sum())
                                                                         / abs(ga64[-1].sum())),
                                              mean_stress_max_abs_err=float(np.abs(sl - s64).max()),
-                                             step_roofline_frac=step_bytes(w.ns, w.P, False, False, True)
+                                             step_roofline_frac=step_bytes(w.eps, w.P, False, False, True)
                                              * rl["steps_per_s"] / 8e12)
         del xl
         area64, area32 = ga64[-1].sum() * w.P, ga32[-1].sum() * w.P
@@ -208,8 +210,8 @@ def main():
                     "slipped_area_fp64": float(area64), "slipped_area_rel_err": float(abs(area32 - area64) / abs(area64)),
                     "mean_stress_max_abs_err": float(np.abs(s32 - s64).max()),
                     "mean_stress_fp64": s64.tolist(),
-                    "step_roofline_frac_mixed": step_bytes(w.ns, w.P, False, True) * r32["steps_per_s"] / 8e12,
-                    "step_roofline_frac_fp64": step_bytes(w.ns, w.P, True, False) * r64["steps_per_s"] / 8e12})
+                    "step_roofline_frac_mixed": step_bytes(w.eps, w.P, False, True) * r32["steps_per_s"] / 8e12,
+                    "step_roofline_frac_fp64": step_bytes(w.eps, w.P, True, False) * r64["steps_per_s"] / 8e12})
     elif a.config == "c3":
         w = C.c3(count=a.count)
         steps = a.steps or w.steps
@@ -241,12 +243,12 @@ def main():
         pts = w.total_points()
         res["mixed_lean"] = dict(rl, speedup=rl["steps_per_s"] / r64["steps_per_s"], xi_max_abs_err=lxerr,
                                  slipped_area_max_rel_err=laerr,
-                                 step_roofline_frac=step_bytes(3, pts, False, False, True) * rl["steps_per_s"] / 8e12)
+                                 step_roofline_frac=step_bytes(w.eps, pts, False, False, True) * rl["steps_per_s"] / 8e12)
         res.update({"count": w.count, "ns": w.ns, "total_points": pts, "steps": steps,
                     "mixed": r32, "fp64": r64, "speedup": r32["steps_per_s"] / r64["steps_per_s"],
                     "xi_max_abs_err": xerr, "slipped_area_max_rel_err": aerr,
-                    "step_roofline_frac_mixed": step_bytes(3, pts, False, False) * r32["steps_per_s"] / 8e12,
-                    "step_roofline_frac_fp64": step_bytes(3, pts, True, False) * r64["steps_per_s"] / 8e12})
+                    "step_roofline_frac_mixed": step_bytes(w.eps, pts, False, False) * r32["steps_per_s"] / 8e12,
+                    "step_roofline_frac_fp64": step_bytes(w.eps, pts, True, False) * r64["steps_per_s"] / 8e12})
     else:
         w = C.c4(steps=a.steps or 5000)
         steps = w.steps
@@ -274,8 +276,8 @@ def main():
                     "mixed_recompute": r32, "fp64_recompute": r64,
                     "stored_vs_recompute_window": {"steps": win, "mixed_stored_steps_per_s": rs["steps_per_s"],
                                                    "mixed_recompute_steps_per_s": rr["steps_per_s"],
-                                                   "stored_GB_s": step_bytes(3, w.P, False, True) * rs["steps_per_s"] / 1e9,
-                                                   "recompute_GB_s": step_bytes(3, w.P, False, False) * rr["steps_per_s"] / 1e9},
+                                                   "stored_GB_s": step_bytes(w.eps, w.P, False, True) * rs["steps_per_s"] / 1e9,
+                                                   "recompute_GB_s": step_bytes(w.eps, w.P, False, False) * rr["steps_per_s"] / 1e9},
                     "xi_max_abs_err": float(np.abs(x32 - x64).max()),
                     "stress_strain_max_abs_err": {"avesigma": float(curve_err), "aveps": float(ceps_err)},
                     "curve_fp64": c64, "curve_mixed": c32})
