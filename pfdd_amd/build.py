@@ -27,7 +27,8 @@ HIP_FLAGS = ["-O3", "-std=c++17", f"--offload-arch={ARCH}", "-fPIC", "-Wall", "-
 # component count and kind, in parallel with the rest
 HIP_UNITS = [("pfdd_api.hip", "pfdd_api.hip.o", [])] + [
     ("pfdd_reduced.hip", f"pfdd_reduced_{k}{r}.o", [f"-DPFDD_RED_R={r}", f"-DPFDD_RED_KIND={k}"])
-    for k in range(4) for r in range(1, 7)] + [("pfdd_reduced.hip", "pfdd_reduced_4.o", ["-DPFDD_RED_KIND=4"])]
+    for k in range(4) for r in range(1, 7)] + [
+    ("pfdd_reduced.hip", f"pfdd_reduced_{k}.o", [f"-DPFDD_RED_KIND={k}"]) for k in (4, 5, 6)]
 C_SOURCES = ["pfdd_setup.c"]
 
 

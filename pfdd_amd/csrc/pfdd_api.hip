@@ -125,6 +125,7 @@ struct pfdd_ctx {
   // the reduced basis (pfdd_reduced.hpp)
   int red = 0;               // 1: the GL steps run in the reduced basis
   int red_R = 0;             // its components
+  int red_plane = 0;         // 1: with the plane kernel
   int red_extra = 0;         // 1: W holds the prologue's extra force, for the next step's update
   RedArgs ra{};
   void* Wr = nullptr;        // cx<T> [B][P][R], allocated with the first plan that uses it
@@ -741,6 +742,28 @@ int red_pass2(pfdd_ctx* c, int sign, const FoldJob& fold = FoldJob{}) {
   return hipPeekAtLastError() == hipSuccess ? PFDD_OK : PFDD_E_HIP;
 }
 
+// Both N2 passes and the column kernel in one launch (c->red_plane).
+template <typename T>
+int red_plane(pfdd_ctx* c, const FinishJob& fin) {
+  RedPlaneLaunch<T> q{};
+  q.W = (cx<T>*)c->Wr;
+  q.ec = c->ec + 1;
+  q.Kst = (const T*)c->Kst;
+  q.n3 = c->p.n3;
+  q.R = c->red_R;
+  q.tw1 = tw_of<T>(c->tw[0]);
+  q.tw2 = tw_of<T>(c->tw[1]);
+  q.batch = (unsigned)c->B;
+  q.fin = fin;
+  q.stream = c->stream;
+  bool ok;
+  if constexpr (sizeof(T) == 8) ok = red_plane_d(q, c->p.n1, c->p.n2);
+  else ok = red_plane_f(q, c->p.n1, c->p.n2);
+  tap(c, PFDD_STAGE_CONTRACT);
+  if (!ok) return PFDD_E_RADIX;
+  return hipPeekAtLastError() == hipSuccess ? PFDD_OK : PFDD_E_HIP;
+}
+
 // The step: the sums of the row kernel's block sums ride along with the N2
 // pass and the column kernel, except that k_finish_sums runs by itself while
 // a point list is set (the step then reports a reduction launch, as with the
@@ -758,13 +781,14 @@ int red_step(pfdd_ctx* c) {
     fin.in = fold.out;
     fin.nblk = FOLD;
   }
-  if ((rc = red_pass2<T>(c, PFDD_FORWARD, fold))) return rc;
+  if (!c->red_plane && (rc = red_pass2<T>(c, PFDD_FORWARD, fold))) return rc;
   if (c->nline > 0) {
     hipLaunchKernelGGL(k_finish_sums, dim3(1), dim3(FIN_THREADS), 0, c->stream, fin.in, c->F, fin.nblk, c->S, c->hist,
                        c->step_ctr);
     tap(c, PFDD_STAGE_FINISH);
     fin.in = nullptr;
   }
+  if (c->red_plane) return red_plane<T>(c, fin);
   if ((rc = red_col<T>(c, fin))) return rc;
   return red_pass2<T>(c, PFDD_BACKWARD);
 }
@@ -1411,7 +1435,7 @@ int apply_plan(pfdd_ctx* c, int plan) {
     c->prologue_done = 0;
     return PFDD_OK;
   }
-  c->red = 0;
+  c->red = c->red_plane = 0;
   if (auto_reduced(c, plan) && ensure_reduced(c)) {
     c->r4 = 0;
     c->row_tile = c->c3_tile = 0;
@@ -1420,6 +1444,8 @@ int apply_plan(pfdd_ctx* c, int plan) {
     const int rows = red_row_rows(c->fp64 != 0, p.n3, c->red_R, S);
     c->row_nblk = (p.n1 * p.n2 + rows - 1) / rows;
     c->red = 1;
+    c->red_plane = plane_fits(c->fp64 != 0, p.n1, p.n2, c->red_R) && !folds(c) &&
+                   plane_faster(p.n1, p.n2, c->red_R, (long)p.n3 * c->B);
     drop_graph(c);
     c->plan = plan;
     c->prologue_done = 0;
@@ -2418,7 +2444,7 @@ extern "C" int pfdd_step_plan(const pfdd_ctx* c, int* launches) {
   const bool r = c->row_tile > 0 || c->plane || c->red, k3 = c->c3_tile > 0 || c->red;
   launches[PFDD_STAGE_UPDATE] = 1;
   launches[PFDD_STAGE_FFT_AXIS3] = r ? 0 : 2;
-  launches[PFDD_STAGE_FFT_AXIS2] = c->plane ? 0 : 2;
+  launches[PFDD_STAGE_FFT_AXIS2] = c->plane || c->red_plane ? 0 : 2;
   launches[PFDD_STAGE_FFT_AXIS1] = k3 ? 0 : 2;
   launches[PFDD_STAGE_CONTRACT] = 1;
   launches[PFDD_STAGE_STEP] = 0;

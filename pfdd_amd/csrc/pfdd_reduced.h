@@ -87,6 +87,31 @@ template <typename T> struct RedPass2Launch {
   FoldJob fold;
   hipStream_t stream;
 };
+// The plane kernel (k_plane_red): its limits, its launch for planes within
+// them, and where it is the faster form: a block walks its plane alone, so that
+// large planes lose when there are few of them (us a step, three kernels
+// against it; components x planes: 2048 x 32 17.9 and 17.6, 3072 x 32 18.5 and
+// 21.2, 5120 x 64 25.4 and 26.7, but 2048 x 128 27.2 and 23.1, 4096 x 128 28.7
+// and 23.4, 3072 x 512 68 and 50).
+constexpr int PLANE_MAX_POINTS = 1024;
+inline bool plane_faster(int n1, int n2, int R, long planes) { return n1 * n2 * R <= 2048 || planes >= 128; }
+constexpr int plane_max_threads(bool fp64) { return fp64 ? 512 : 768; }
+constexpr int plane_rl(bool fp64, int n1) { return fp64 && n1 >= 128 ? 8 : RED_RL; }
+int plane_threads(bool fp64, int n1, int n2, int R);
+size_t plane_lds(bool fp64, int n1, int n2, int R);
+bool plane_fits(bool fp64, int n1, int n2, int R);
+template <typename T> struct RedPlaneLaunch {
+  cx<T>* W;
+  const ElasticConsts* ec;
+  const T* Kst;
+  int n3, R;
+  const cx<T>*tw1, *tw2;
+  unsigned batch;
+  FinishJob fin;
+  hipStream_t stream;
+};
+bool red_plane_d(const RedPlaneLaunch<double>&, int n1, int n2);
+bool red_plane_f(const RedPlaneLaunch<float>&, int n1, int n2);
 bool red_pass2_d(const RedPass2Launch<double>&, int n2);
 bool red_pass2_f(const RedPass2Launch<float>&, int n2);
 bool red_pass2_attr(int n2);  // LDS limits of both, once per context

@@ -508,8 +508,8 @@ __device__ __forceinline__ void wave_sums4(const FinishJob& j, int f0, double (&
 }
 // (The history row lies in host memory: it is written, never read back.)
 constexpr int FINISH_LDS = 64;  // fields whose sums the block holds in LDS
-template <int NT> __device__ __forceinline__ void finish_block(const FinishJob& j) {
-  constexpr int NW = NT / 64;
+__device__ __forceinline__ void finish_block(const FinishJob& j) {
+  const int NT = blockDim.x, NW = NT / 64;
   __shared__ double fsum[FINISH_LDS];
   const int ninst = j.F / j.S, w = threadIdx.x >> 6;
   const bool lane0 = (threadIdx.x & 63) == 0;
@@ -636,7 +636,7 @@ k_col_red(cx<T>* __restrict__ W, const ElasticConsts* __restrict__ ec, const T* 
   __shared__ cx<T> sm[NPEN * LD];
   __shared__ cx<T> twl[N];
   if ((int)blockIdx.x >= blocks) {
-    finish_block<NT>(fin);
+    finish_block(fin);
     return;
   }
   const int t = threadIdx.x;
@@ -702,6 +702,76 @@ k_pass2_red(cx<T>* __restrict__ data, int inner, int blocks, T sign, const cx<T>
   const LdsPencils<T> l{sm, LD};
   fft_pencils<T, N, 1, RED_RL>(g, l, g, (int)threadIdx.x % TILE, 1 << 30, np, (int)threadIdx.x / TILE, sign, twl,
                        [&] { ts.store(twl); });
+}
+
+// ---------------------------------------------------------------- plane kernel
+// One block: the N1 x N2 plane of one i3, all R components, in LDS: forward N2
+// and N1, K(k), inverse N1 and N2 -- the two N2 passes and the column kernel in
+// one launch and one trip through memory, with their arithmetic.  On small
+// grids a launch costs 4 to 5 us whatever it does (32x2x32 x 2: 14.2 against
+// 11.1 us a step, 256x2x256 x 3: 29.7 against 21.2); on many planes the two
+// trips count (64 instances of 32^3 x 3: 184 against 119).  Threads:
+// plane_threads(), one pencil share each.  grid = instances x N3, and one
+// block for the sums.
+template <typename T> struct PlaneN2 {  // N2 pencils of the plane in LDS: pencil p = n1 R + c
+  cx<T>* sm;
+  int R, ld;
+  static constexpr bool in_lds = true;
+  __device__ __forceinline__ cx<T>* at(int p, int i) const { return sm + (i * R + p % R) * ld + p / R; }
+  __device__ __forceinline__ cx<T> load(int p, int i) const { return *at(p, i); }
+  __device__ __forceinline__ void store(int p, int i, cx<T> v) const { *at(p, i) = v; }
+};
+template <typename T, int N1, int N2>
+__global__ void __launch_bounds__(plane_max_threads(sizeof(T) == 8))
+k_plane_red(cx<T>* __restrict__ W, const ElasticConsts* __restrict__ ec, const T* __restrict__ Kst, int n3, int R,
+            int blocks, const cx<T>* __restrict__ tw1, const cx<T>* __restrict__ tw2, const FinishJob fin) {
+  constexpr int LD = pitch<N1>(), RL1 = plane_rl(sizeof(T) == 8, N1), P = N1 * N2;
+  constexpr int TPP1 = make_plan(N1, RL1).tpp, TPP2 = make_plan(N2, RED_RL).tpp;
+  extern __shared__ unsigned char lds_raw[];  // plane_lds()
+  cx<T>* sm = reinterpret_cast<cx<T>*>(lds_raw);
+  cx<T>*twl1 = sm + N2 * R * LD, *twl2 = twl1 + N1;
+  if ((int)blockIdx.x >= blocks) {
+    finish_block(fin);
+    return;
+  }
+  const int t = threadIdx.x;
+  const int b = (int)xcd_tile(blockIdx.x, blocks), inst = b / n3, i3 = b - inst * n3;
+  cx<T>* base = W + ((long)inst * P * n3 + i3) * R;
+  const cx<T> w1 = tw1[t < N1 ? t : N1 - 1], w2 = tw2[t < N2 ? t : N2 - 1];
+  const int np2 = N1 * R, p2 = t % np2, q2 = t / np2;
+  const int np1 = N2 * R, p1 = t % np1, q1 = t / np1;
+  const int pen2 = q2 < TPP2 ? p2 : 1 << 30, pen1 = q1 < TPP1 ? p1 : 1 << 30;
+  const StridedPencil<T> g{base + (long)(p2 / R) * N2 * n3 * R + p2 % R, (long)n3 * R};
+  const PlaneN2<T> l2{sm, R, LD};
+  const LdsPencils<T> l1{sm, LD};
+  fft_pencils<T, N2, 1, RED_RL>(g, l2, l2, pen2, 1 << 30, np2, q2, (T)-1, twl2, [&] {
+    if (t < N1) twl1[t] = w1;
+    if (t < N2) twl2[t] = w2;
+  });
+  fft_pencils<T, N1, 1, RL1>(l1, l1, l1, pen1, 1 << 30, np1, q1, (T)-1, twl1);
+  for (int e = t; e < P; e += blockDim.x) {
+    const int i1 = e % N1, i2 = e / N1;
+    const long k = ((long)i1 * N2 + i2) * n3 + i3;
+    cx<T>* io = sm + i2 * R * LD + i1;
+    double f[3], gr[6];
+    bool nz = false;
+    if (!Kst) {
+      kvec(k, ec, f);
+      nz = green6_rcp(f, ec, gr);
+    }
+    switch (R) {
+#define PFDD_R(RR)                                                                       \
+  case RR:                                                                               \
+    if (Kst) contract_stored_lds<T, RR>(io, LD, Kst + k * (RR * (RR + 1) / 2));          \
+    else contract_stress_form_lds<T, RR>(io, LD, ec, f, gr, nz);                         \
+    break;
+      PFDD_R(1) PFDD_R(2) PFDD_R(3) PFDD_R(4) PFDD_R(5) PFDD_R(6)
+#undef PFDD_R
+    }
+  }
+  __syncthreads();
+  fft_pencils<T, N1, 1, RL1>(l1, l1, l1, pen1, 1 << 30, np1, q1, (T)1, twl1);
+  fft_pencils<T, N2, 1, RED_RL>(l2, l2, g, pen2, 1 << 30, np2, q2, (T)1, twl2);
 }
 
 }  // namespace pfdd

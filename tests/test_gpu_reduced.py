@@ -173,3 +173,36 @@ def test_classes_on_parallel_branches(sizes):
                 gs.append(c.gl_steps(n)[0])
             assert np.array_equal(c.download_xi(), got[i]), i
         assert np.array_equal(np.concatenate(gs), np.concatenate(g)[:, i]), i
+
+
+@pytest.mark.parametrize("prec", PRECS)
+@pytest.mark.parametrize("n1", sorted(SHORT + FUSED))
+def test_both_sides_of_the_plane_kernel(n1, prec):
+    """The largest N2 whose N1 x N2 plane is transformed in one launch, and
+    the smallest that takes the N2 passes and the column kernel."""
+    for ns, n3 in ((3, 8), (12, 3)):
+        last = None
+        for n2 in sorted(SHORT + FUSED):
+            w = C.small_fcc((n1, n2, n3), ns=ns, nloops=3)
+            with pa.Context(w.params(prec)) as c:
+                plane = c.step_plan()[pa.STAGE_FFT_AXIS2] == 0
+            if not plane:
+                break
+            last = w
+        assert not plane
+        check(w, prec)
+        if last is not None:
+            check(last, prec)
+        check(w, prec, bmode=pa.B_STORED)
+        if last is not None:
+            check(last, prec, bmode=pa.B_STORED)
+
+
+@pytest.mark.parametrize("prec", PRECS)
+@pytest.mark.parametrize("n1,n2,ns", [(32, 32, 4), (24, 32, 5), (8, 96, 5), (48, 16, 4), (16, 32, 12)])
+def test_large_planes(n1, n2, ns, prec):
+    """Planes that take one launch only when there are many of them."""
+    w = C.small_fcc((n1, n2, 128), ns=ns, nloops=3)
+    with pa.Context(w.params(prec)) as c:
+        assert c.step_plan()[pa.STAGE_FFT_AXIS2] == 0
+    check(w, prec)
