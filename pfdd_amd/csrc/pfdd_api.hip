@@ -1387,6 +1387,11 @@ bool ensure_reduced(pfdd_ctx* c) {
   void* wr = dev_alloc<char>(csz * c->B * c->P * R, bytes);
   void* ks = c->stored && wr ? dev_alloc<char>(csz / 2 * (R * (R + 1) / 2) * c->P, bytes) : nullptr;
   bool ok = wr && (ks || !c->stored) && red_pass2_attr(c->p.n2);
+  switch (R) {
+#define PFDD_R(RR) case RR: ok = ok && red_col_attr##RR(c->p.n1); break;
+    PFDD_R(1) PFDD_R(2) PFDD_R(3) PFDD_R(4) PFDD_R(5) PFDD_R(6)
+#undef PFDD_R
+  }
   if (ok && ks) {
     switch (R) {
 #define PFDD_R(RR)                                                             \

@@ -122,6 +122,7 @@ bool red_pass2_attr(int n2);  // LDS limits of both, once per context
   bool red_row_l##R(const RedRowLaunch<float>&, MasterF32L, int n3);      \
   bool red_col_d##R(const RedColLaunch<double>&, int n1);                 \
   bool red_col_f##R(const RedColLaunch<float>&, int n1);                  \
+  bool red_col_attr##R(int n1);  /* LDS limits of both, once per context */ \
   void red_build_d##R(double* Kst, const ElasticConsts* ec, long P, hipStream_t);  \
   void red_build_f##R(float* Kst, const ElasticConsts* ec, long P, hipStream_t);
 PFDD_RED_DECL(1) PFDD_RED_DECL(2) PFDD_RED_DECL(3) PFDD_RED_DECL(4) PFDD_RED_DECL(5) PFDD_RED_DECL(6)

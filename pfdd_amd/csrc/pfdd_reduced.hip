@@ -52,11 +52,20 @@ template <typename T, int N> void col(const RedColLaunch<T>& q) {
   const int blocks = (int)((q.P / N + K::TC - 1) / K::TC * q.batch);
   const dim3 grid((unsigned)(blocks + (q.fin.in ? 1 : 0)));
   if (q.Kst)
-    hipLaunchKernelGGL((k_col_red<T, N, R, true>), grid, dim3(K::NT), 0, q.stream, q.W, q.ec, q.Kst, q.P, blocks, q.tw,
+    hipLaunchKernelGGL((k_col_red<T, N, R, true>), grid, dim3(K::NT), K::LDS, q.stream, q.W, q.ec, q.Kst, q.P, blocks, q.tw,
                        q.fin);
   else
-    hipLaunchKernelGGL((k_col_red<T, N, R, false>), grid, dim3(K::NT), 0, q.stream, q.W, q.ec, q.Kst, q.P, blocks, q.tw,
+    hipLaunchKernelGGL((k_col_red<T, N, R, false>), grid, dim3(K::NT), K::LDS, q.stream, q.W, q.ec, q.Kst, q.P, blocks, q.tw,
                        q.fin);
+}
+// The LDS limit of the tiles wider than 64 KB.
+template <typename T, int N> bool col_attr() {
+  constexpr int L = (int)ColRed<T, N, R>::LDS;
+  if constexpr (L <= 64 * 1024) return true;
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(&k_col_red<T, N, R, true>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, L) == hipSuccess &&
+         hipFuncSetAttribute(reinterpret_cast<const void*>(&k_col_red<T, N, R, false>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, L) == hipSuccess;
 }
 template <typename T> void build(T* Kst, const ElasticConsts* ec, long P, hipStream_t st) {
   hipLaunchKernelGGL((k_build_K<T, R>), dim3((unsigned)((P + 255) / 256)), dim3(256), 0, st, Kst, ec, P);
@@ -140,6 +149,9 @@ bool PFDD_CAT(red_row_l, PFDD_RED_R)(const RedRowLaunch<float>& q, MasterF32L xi
 #elif PFDD_RED_KIND == 3
 bool PFDD_CAT(red_col_d, PFDD_RED_R)(const RedColLaunch<double>& q, int n1) { return col_any(q, n1); }
 bool PFDD_CAT(red_col_f, PFDD_RED_R)(const RedColLaunch<float>& q, int n1) { return col_any(q, n1); }
+bool PFDD_CAT(red_col_attr, PFDD_RED_R)(int n1) {
+  return n1 != 512 || (col_attr<double, 512>() && col_attr<float, 512>());
+}
 void PFDD_CAT(red_build_d, PFDD_RED_R)(double* K, const ElasticConsts* ec, long P, hipStream_t st) { build(K, ec, P, st); }
 void PFDD_CAT(red_build_f, PFDD_RED_R)(float* K, const ElasticConsts* ec, long P, hipStream_t st) { build(K, ec, P, st); }
 #elif PFDD_RED_KIND == 4

@@ -438,24 +438,29 @@ k_row_red_n(cx<T>* __restrict__ W, M xi, const RedArgs a, const RedOpt<T> o, con
 
 // ---------------------------------------------------------------- column kernel
 // Columns per block TC: row segments (R TC complex) of 128 to 192 bytes where
-// 48 KB of LDS allow it; about 256 k-points where N < 32.
+// 48 KB of LDS allow it; about 256 k-points where N < 32.  At 512, whose rows
+// lie megabytes apart, 72 KB: two blocks a CU with segments of 128 bytes beat
+// four with 64 (512x128x512 x 3 FP64 669 against 821 us, mixed 445 against 462;
+// at 384 they do not: 384x96x384 x 3 355 against 323).
 // Radix limit: two passes (16) are faster in FP32 and, in FP64, at 48 and 96;
 // FP64's radix-16 pass at 128, 192 and 256 leaves half the lanes idle and
 // measured slower (128^3 x 3: 51 against 42 us, 256x256x192 x 3: 279 against 220).
 template <typename T, int N, int R> struct ColRed {
   static constexpr int RL = sizeof(T) == 8 && N >= 128 ? 8 : RED_RL;
   static constexpr int TPP = make_plan(N, RL).tpp, LD = pitch<N>();
-  static constexpr size_t CSZ = sizeof(cx<T>);
+  static constexpr size_t CSZ = sizeof(cx<T>), LIMIT = (N >= 512 ? 72 : 48) * 1024;
   static constexpr int tc() {
     int t = 1;
     if (N < 32) {
       while (N * t * 2 <= 256 && t * 2 * R * TPP <= 512) t *= 2;
       return t;
     }
-    while (t * 2 * R * CSZ <= 192 && (size_t)t * 2 * R * LD * CSZ <= 48 * 1024 && t * 2 * R * TPP <= 1024) t *= 2;
+    while (t * 2 * R * CSZ <= 192 && (size_t)t * 2 * R * LD * CSZ <= LIMIT && t * 2 * R * TPP <= 1024) t *= 2;
     return t;
   }
-  static constexpr int TC = tc(), NPEN = R * TC, LANES = (NPEN * TPP + 63) / 64 * 64;
+  static constexpr int TC = tc(), NPEN = R * TC;
+  static constexpr size_t LDS = ((size_t)NPEN * LD + N) * CSZ;  // tile and twiddles
+  static constexpr int LANES = (NPEN * TPP + 63) / 64 * 64;
   static constexpr int PTS = N * TC < 512 ? N * TC : 512;
   static constexpr int NT = LANES > PTS ? LANES : (PTS + 63) / 64 * 64;
   static constexpr int KPT = (N * TC + NT - 1) / NT;  // k-points per thread
@@ -633,8 +638,9 @@ k_col_red(cx<T>* __restrict__ W, const ElasticConsts* __restrict__ ec, const T* 
           const cx<T>* __restrict__ tw, const FinishJob fin) {
   using K = ColRed<T, N, R>;
   constexpr int NT = K::NT, LD = K::LD, TPP = K::TPP, TC = K::TC, NPEN = K::NPEN;
-  __shared__ cx<T> sm[NPEN * LD];
-  __shared__ cx<T> twl[N];
+  extern __shared__ unsigned char lds_raw[];  // K::LDS
+  cx<T>* sm = reinterpret_cast<cx<T>*>(lds_raw);
+  cx<T>* twl = sm + NPEN * LD;
   if ((int)blockIdx.x >= blocks) {
     finish_block(fin);
     return;

@@ -206,3 +206,12 @@ def test_large_planes(n1, n2, ns, prec):
     with pa.Context(w.params(prec)) as c:
         assert c.step_plan()[pa.STAGE_FFT_AXIS2] == 0
     check(w, prec)
+
+
+@pytest.mark.parametrize("prec", PRECS)
+@pytest.mark.parametrize("n1", [384, 512])
+@pytest.mark.parametrize("ns", [1, 3, 4, 5, 6])
+def test_wide_column_tiles(n1, ns, prec):
+    """Column counts that are no multiple of the tiles at the longest N1."""
+    check(C.small_fcc((n1, 3, 6), ns=ns, nloops=2), prec)
+    check(C.small_fcc((n1, 3, 6), ns=ns, nloops=2), prec, bmode=pa.B_STORED)
